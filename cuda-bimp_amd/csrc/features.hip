@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 
 #include "../../include/bimp_hip.h"
 
@@ -59,13 +60,20 @@ __global__ void __launch_bounds__(64) k_color_features(const float* __restrict__
 }
 
 // ------------------------------------------------------------------ 2-NN matching
-// A workgroup of 256 threads owns 64 query rows and walks every train row in tiles of 64.
-// Thread (ty, tx) accumulates the 4 x 4 squared distances of queries 4ty.. and trains
-// 4tx.. of a tile over the dimensions, staged through LDS 32 at a time (both tiles stored
-// dimension-major, so a thread reads one float4 of each per dimension); it keeps the best two
-// (distance, index) of its 4 queries over its train columns, and the 16 threads of a query
-// row merge theirs at the end.  Ties go to the lower train index.
-constexpr int KQ = 64, KT = 64, DC = 32, PADQ = KQ + 4;
+// A workgroup of 16 x 16 threads owns 16R query rows and walks the tiles of 16R train rows of
+// its slice of the train set (blockIdx.y); thread (ty, tx) accumulates the R x R squared
+// distances of its queries and trains over the dimensions, in order, and keeps the best two
+// (distance, index) of each of its queries.  Both tiles pass through LDS kDC dimensions at a
+// time, dimension-major, in two buffers: the next piece is loaded into registers while the
+// current one is used, one barrier per piece.
+//
+// Bound: FP32 VALU, one subtraction and one fma per query, train and dimension (no packed
+// FP32; the matrix cores' |q|^2 + |t|^2 - 2qt would lose the small distances' digits): 8000 x
+// 8000 x 152 takes 0.44 ms back to back, no more than these operations alone take at 2.4 GHz.
+// R = 4 takes two 16-byte LDS reads per 32 of them.  Before, one
+// workgroup walked the whole train set for its 64 queries, in one LDS buffer: 125 workgroups
+// for 8000 queries, 3.66 ms; 517 x 433 x 152 took 177 us on 9 workgroups, now 16 us.
+constexpr int kDC = 16;
 
 struct Best2 {
     float d0, d1;
@@ -88,73 +96,236 @@ __device__ __forceinline__ void insert(Best2& b, float d, int i) {
     }
 }
 
+// Order-preserving key of a candidate: squared distances are non-negative, so their bits order
+// as unsigned integers; the index breaks ties toward the lower one.  No candidate: +inf, ~0.
+typedef unsigned long long u64;
+constexpr u64 kNoKey = ((u64)0x7f800000u << 32) | 0xffffffffu;
+__device__ __forceinline__ u64 key_of(float d, int i) {
+    return ((u64)__float_as_uint(d) << 32) | (unsigned)i;
+}
+
+// Slices of the train set meet in the outputs: query i's best key sits in its idx2 pair, its
+// second best in its dist2 pair (8 bytes each, 8-byte aligned).  The displaced key, or the
+// offered one if it does not displace any, goes on to the second slot, so that once all have
+// been offered the slots hold the two smallest in any order of arrival.
+__device__ __forceinline__ void offer(u64* best, u64* second, u64 k) {
+    const u64 old = atomicMin(best, k);
+    const u64 rest = old < k ? k : old;
+    if (rest < kNoKey) atomicMin(second, rest);
+}
+
+__global__ void k_knn2_init(u64* __restrict__ best, u64* __restrict__ second, int nq) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nq) best[i] = second[i] = kNoKey;
+}
+
+__global__ void k_knn2_unpack(int* __restrict__ idx2, float* __restrict__ dist2, int nq) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nq) return;
+    const u64 a = *reinterpret_cast<const u64*>(idx2 + 2 * (size_t)i);
+    const u64 b = *reinterpret_cast<const u64*>(dist2 + 2 * (size_t)i);
+    idx2[2 * (size_t)i] = (int)(unsigned)a;
+    idx2[2 * (size_t)i + 1] = (int)(unsigned)b;
+    dist2[2 * (size_t)i] = sqrtf(__uint_as_float((unsigned)(a >> 32)));
+    dist2[2 * (size_t)i + 1] = sqrtf(__uint_as_float((unsigned)(b >> 32)));
+}
+
+template <int R>
+__device__ __forceinline__ void read_rows(const float* __restrict__ row, int t, float (&v)[R]) {
+    if constexpr (R == 2) {
+        const float2 a = *reinterpret_cast<const float2*>(row + 2 * t);
+        v[0] = a.x;
+        v[1] = a.y;
+    } else {
+        const float4 a = *reinterpret_cast<const float4*>(row + 4 * t);
+        v[0] = a.x;
+        v[1] = a.y;
+        v[2] = a.z;
+        v[3] = a.w;
+    }
+}
+
+// VEC: rows are 16-byte aligned (base and stride), so four dimensions load at once.
+// ATOMIC: several slices per query (gridDim.y > 1) meet in the outputs' key slots.
+template <int R, bool VEC, bool ATOMIC>
 __global__ void __launch_bounds__(256) k_knn2(const float* __restrict__ q, int nq, int qld,
                                               const float* __restrict__ t, int nt, int tld,
-                                              int dim, int* __restrict__ idx2,
-                                              float* __restrict__ dist2) {
-    __shared__ __align__(16) float qs[DC][PADQ];
-    __shared__ __align__(16) float ts[DC][PADQ];
-    __shared__ Best2 part[KQ][17];
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int q0 = blockIdx.x * KQ;
-    Best2 b[4];
+                                              int dim, int tiles_per_slice,
+                                              int* __restrict__ idx2, float* __restrict__ dist2) {
+    constexpr int K = 16 * R, PAD = K + 4;         // PAD = 4 (mod 16) words: the transposing
+    constexpr int NV = K * kDC / 4;                // stores spread over the banks
+    constexpr int PER = (NV + 255) / 256;          // float4 a thread stages per operand
+    __shared__ __align__(16) float qs[2][kDC][PAD];
+    __shared__ __align__(16) float ts[2][kDC][PAD];
+    const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
+    const int q0 = blockIdx.x * K;
+    const int ntiles = (nt + K - 1) / K;
+    const int tile0 = blockIdx.y * tiles_per_slice;
+    const int tile1 = min(ntiles, tile0 + tiles_per_slice);
+    const int nc = (dim + kDC - 1) / kDC;
+    Best2 b[R];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) b[r] = Best2{INFINITY, INFINITY, -1, -1};
-    for (int t0 = 0; t0 < nt; t0 += KT) {
-        float acc[4][4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[r][c] = 0.f;
-        for (int d0 = 0; d0 < dim; d0 += DC) {
-            __syncthreads();
-            for (int e = threadIdx.x; e < KQ * DC; e += 256) {
-                const int r = e / DC, d = e % DC;
-                const bool dv = d0 + d < dim;
-                qs[d][r] = (dv && q0 + r < nq) ? q[(size_t)(q0 + r) * qld + d0 + d] : 0.f;
-                ts[d][r] = (dv && t0 + r < nt) ? t[(size_t)(t0 + r) * tld + d0 + d] : 0.f;
-            }
-            __syncthreads();
-            const int dn = min(DC, dim - d0);
-            for (int d = 0; d < dn; ++d) {
-                const float4 qa = *reinterpret_cast<const float4*>(&qs[d][4 * ty]);
-                const float4 ta = *reinterpret_cast<const float4*>(&ts[d][4 * tx]);
-                const float qv[4] = {qa.x, qa.y, qa.z, qa.w};
-                const float tv[4] = {ta.x, ta.y, ta.z, ta.w};
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const float df = qv[r] - tv[c];
-                        acc[r][c] = fmaf(df, df, acc[r][c]);
-                    }
+    for (int r = 0; r < R; ++r) b[r] = Best2{INFINITY, INFINITY, -1, -1};
+
+    float4 pq[PER], pt[PER];
+    auto load = [&](const float* __restrict__ base, int row, int rows, int ld, int d) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (row < rows && d < dim) {
+            const float* p = base + (size_t)row * ld + d;
+            if (VEC && d + 4 <= dim) {
+                v = *reinterpret_cast<const float4*>(p);
+            } else {
+                v.x = p[0];
+                if (d + 1 < dim) v.y = p[1];
+                if (d + 2 < dim) v.z = p[2];
+                if (d + 3 < dim) v.w = p[3];
             }
         }
+        return v;
+    };
+    auto fetch = [&](int tile, int c) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int ti = t0 + 4 * tx + c;
-            if (ti >= nt) continue;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) insert(b[r], acc[r][c], ti);
+        for (int k = 0; k < PER; ++k) {
+            const int e = tid + 256 * k, r = e / (kDC / 4), d = c * kDC + 4 * (e % (kDC / 4));
+            if (NV % 256 == 0 || e < NV) {
+                pq[k] = load(q, q0 + r, nq, qld, d);
+                pt[k] = load(t, tile * K + r, nt, tld, d);
+            }
         }
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int e = tid + 256 * k, r = e / (kDC / 4), d = 4 * (e % (kDC / 4));
+            if (NV % 256 == 0 || e < NV) {
+                qs[buf][d][r] = pq[k].x;
+                qs[buf][d + 1][r] = pq[k].y;
+                qs[buf][d + 2][r] = pq[k].z;
+                qs[buf][d + 3][r] = pq[k].w;
+                ts[buf][d][r] = pt[k].x;
+                ts[buf][d + 1][r] = pt[k].y;
+                ts[buf][d + 2][r] = pt[k].z;
+                ts[buf][d + 3][r] = pt[k].w;
+            }
+        }
+    };
+
+    float acc[R][R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < R; ++c) acc[r][c] = 0.f;
+    auto step = [&](int buf, int d) {
+        float qv[R], tv[R];
+        read_rows<R>(qs[buf][d], ty, qv);
+        read_rows<R>(ts[buf][d], tx, tv);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int c = 0; c < R; ++c) {
+                const float df = qv[r] - tv[c];
+                acc[r][c] = fmaf(df, df, acc[r][c]);
+            }
+    };
+
+    if (tile0 < tile1) {
+        fetch(tile0, 0);
+        put(0);
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) part[4 * ty + r][tx] = b[r];
     __syncthreads();
-    if (threadIdx.x < KQ && q0 + (int)threadIdx.x < nq) {
-        const int r = threadIdx.x;
-        Best2 m = part[r][0];
-        for (int k = 1; k < 16; ++k) {
-            const Best2 o = part[r][k];
-            insert(m, o.d0, o.i0);
-            insert(m, o.d1, o.i1);
+    int buf = 0;
+    for (int tile = tile0; tile < tile1; ++tile) {
+        for (int c = 0; c < nc; ++c) {
+            const bool more = c + 1 < nc || tile + 1 < tile1;
+            if (more) fetch(c + 1 < nc ? tile : tile + 1, c + 1 < nc ? c + 1 : 0);
+            if ((c + 1) * kDC <= dim) {
+#pragma unroll 4
+                for (int d = 0; d < kDC; ++d) step(buf, d);
+            } else {
+                for (int d = 0; d < dim - c * kDC; ++d) step(buf, d);
+            }
+            if (more) put(buf ^ 1);  // its readers passed the barrier of the piece before
+            __syncthreads();
+            buf ^= 1;
         }
-        const size_t qi = (size_t)(q0 + r);
-        idx2[2 * qi] = m.i0;
-        idx2[2 * qi + 1] = m.i1;
-        dist2[2 * qi] = sqrtf(m.d0);
-        dist2[2 * qi + 1] = sqrtf(m.d1);
+#pragma unroll
+        for (int c = 0; c < R; ++c) {
+            const int ti = tile * K + R * tx + c;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (ti < nt) insert(b[r], acc[r][c], ti);
+                acc[r][c] = 0.f;
+            }
+        }
     }
+    // the 16 threads of a query row merge their pairs across lanes (a row's threads are 16
+    // consecutive lanes); lane tx = 0 holds the result
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        Best2 m = b[r];
+#pragma unroll
+        for (int sh = 8; sh >= 1; sh >>= 1) {
+            const float d0 = __shfl_xor(m.d0, sh, 16), d1 = __shfl_xor(m.d1, sh, 16);
+            const int i0 = __shfl_xor(m.i0, sh, 16), i1 = __shfl_xor(m.i1, sh, 16);
+            insert(m, d0, i0);
+            insert(m, d1, i1);
+        }
+        const int qi = q0 + R * ty + r;
+        if (tx == 0 && qi < nq) {
+            int* const oi = idx2 + 2 * (size_t)qi;
+            float* const od = dist2 + 2 * (size_t)qi;
+            if constexpr (ATOMIC) {
+                u64* const best = reinterpret_cast<u64*>(oi);
+                u64* const second = reinterpret_cast<u64*>(od);
+                if (m.i0 >= 0) offer(best, second, key_of(m.d0, m.i0));
+                if (m.i1 >= 0) offer(best, second, key_of(m.d1, m.i1));
+            } else {
+                oi[0] = m.i0;
+                oi[1] = m.i1;
+                od[0] = sqrtf(m.d0);
+                od[1] = sqrtf(m.d1);
+            }
+        }
+    }
+}
+
+template <int R, bool VEC>
+void launch_knn2(const float* q, int nq, int qld, const float* t, int nt, int tld, int dim,
+                 int* idx2, float* dist2, hipStream_t s) {
+    constexpr int K = 16 * R;
+    const int ntiles = (nt + K - 1) / K, nqt = (nq + K - 1) / K;
+    // One tile per workgroup up to 4096 workgroups, then slices of several tiles (8000 x 8000:
+    // 32 slices 479 us, 8 slices 552 us; 4000 x 4000: 63 slices 131 us, 8 slices 177 us; 517 x
+    // 433: 14 slices 16 us, one 119 us).  The outputs hold the slices' keys only where they are
+    // 8-byte aligned; otherwise a query has one slice.
+    const bool keys = ((uintptr_t)idx2 | (uintptr_t)dist2) % 8 == 0;
+    int per = std::max(1, ntiles);
+    if (keys) per = std::max(1, (int)(((long)ntiles * nqt + 4095) / 4096));
+    // (a grid's y extent is limited to 65535)
+    per = std::max(per, (ntiles + 65534) / 65535);
+    const dim3 grid(nqt, std::max(1, (ntiles + per - 1) / per));
+    if (grid.y > 1) {
+        u64 *best = reinterpret_cast<u64*>(idx2), *second = reinterpret_cast<u64*>(dist2);
+        k_knn2_init<<<(nq + 255) / 256, 256, 0, s>>>(best, second, nq);
+        k_knn2<R, VEC, true><<<grid, 256, 0, s>>>(q, nq, qld, t, nt, tld, dim, per, idx2, dist2);
+        k_knn2_unpack<<<(nq + 255) / 256, 256, 0, s>>>(idx2, dist2, nq);
+    } else {
+        k_knn2<R, VEC, false><<<grid, 256, 0, s>>>(q, nq, qld, t, nt, tld, dim, per, idx2, dist2);
+    }
+}
+
+template <bool VEC>
+void dispatch_knn2(const float* q, int nq, int qld, const float* t, int nt, int tld, int dim,
+                   int* idx2, float* dist2, hipStream_t s) {
+    // R = 4 where its tiles fill the chip's 256 CUs a few times over (it runs six workgroups
+    // per CU), else R = 2, whose tiles are four times as many: 2000 x 2000 x 152 (1024 tiles of
+    // 64 x 64) 45 us against 57 us with R = 2, 1000 x 1000 (256 tiles) 31 against 22 us.  R = 8
+    // took 525 us against 479 us at 8000 x 8000 (211 VGPRs, two wavefronts per SIMD).
+    const long tiles4 = (long)((nq + 63) / 64) * ((nt + 63) / 64);
+    if (tiles4 >= 768)
+        launch_knn2<4, VEC>(q, nq, qld, t, nt, tld, dim, idx2, dist2, s);
+    else
+        launch_knn2<2, VEC>(q, nq, qld, t, nt, tld, dim, idx2, dist2, s);
 }
 
 }  // namespace
@@ -178,8 +349,14 @@ int bimp_match_knn2(const float* d_query, int nq, int q_ld, const float* d_train
         (nq > 0 && (!d_query || !d_idx2 || !d_dist2)) || (nt > 0 && !d_train))
         return BIMP_E_ARG;
     if (nq == 0) return BIMP_OK;
-    k_knn2<<<(nq + KQ - 1) / KQ, 256, 0, (hipStream_t)stream>>>(d_query, nq, q_ld, d_train, nt,
-                                                                t_ld, dim, d_idx2, d_dist2);
+    const bool vec = q_ld % 4 == 0 && t_ld % 4 == 0 &&
+                     ((uintptr_t)d_query | (uintptr_t)d_train) % 16 == 0;
+    if (vec)
+        dispatch_knn2<true>(d_query, nq, q_ld, d_train, nt, t_ld, dim, d_idx2, d_dist2,
+                            (hipStream_t)stream);
+    else
+        dispatch_knn2<false>(d_query, nq, q_ld, d_train, nt, t_ld, dim, d_idx2, d_dist2,
+                             (hipStream_t)stream);
     return hipGetLastError() == hipSuccess ? BIMP_OK : BIMP_E_DEVICE;
 }
 
