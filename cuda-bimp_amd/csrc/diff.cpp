@@ -19,44 +19,7 @@
 
 #include "../../include/bimp_hip.h"
 #include "bank.hpp"
-#include "kernels.hpp"
-
-namespace bimpk {
-hipError_t diff_prepare(int n);
-hipError_t diff_rows(float2* data, int rows, int n, bool inv, const float2* tw, hipStream_t s);
-hipError_t diff_rows_maps(float2* data, int maps, int per_map, size_t map_stride, int n,
-                          bool inv, const float2* tw, hipStream_t s);
-hipError_t diff_gather_tap_rows(const float2* Z, int kW, int kX, int FH, int FW, float2* Yc,
-                                int nb, hipStream_t s);
-hipError_t diff_cols(float2* data, int n, int w, int batch, bool inv, const float2* tw,
-                     hipStream_t s);
-hipError_t diff_pyr_down(const float* src, int sw, int sh, float* dst, int dw, int dh, int nb,
-                         hipStream_t s);
-hipError_t diff_pyr_down_adj(const float* gdst, int dw, int dh, float* gsrc, int sw, int sh,
-                             int nb, hipStream_t s);
-hipError_t diff_pad(const float* L, int pitch, size_t lstride, int H, int W, int FH, int FW,
-                    int k, float sc, float2* out, int nb, hipStream_t s);
-hipError_t diff_pad_adj(const float2* g, int H, int W, int FH, int FW, int k, float sc,
-                        float* gL, int pitch, size_t lstride, int nb, hipStream_t s);
-hipError_t diff_q_to_g(const float2* Q, int FH, int FW, float invN, float* G, hipStream_t s);
-hipError_t diff_bank_pad(const float* ke, const float* ko, int kW, int kX, int FH, int FW,
-                         float2* out, hipStream_t s);
-hipError_t diff_spec_mul(const float2* D, const float2* Q, float2* Z, size_t n, int nb,
-                         float invN, hipStream_t s);
-hipError_t diff_mag(const float2* Z, float* C, size_t n, hipStream_t s);
-hipError_t diff_cells_adj(const float* C, int FH, int FW, int H, int W, const CellParams& p,
-                          const float* gD, size_t gstride, float* Wm, float* gC, int nb,
-                          hipStream_t s);
-hipError_t diff_grad_z(const float* gC, float2* Z, size_t n, hipStream_t s);
-hipError_t diff_accum_conjq(const float2* Q, const float2* G, float2* out, size_t n, int nb,
-                            float invN, hipStream_t s);
-hipError_t diff_mul_conjd(float2* G, const float2* D, size_t n, int nb, float invN,
-                          hipStream_t s);
-int diff_param_blocks(int kW);
-hipError_t diff_param_partials(const float2* Yc, int kW, int kX, int FW, const float* dK,
-                               float* partials, size_t pstride, int nb, hipStream_t s);
-hipError_t diff_fill(float* p, size_t n, hipStream_t s);
-}  // namespace bimpk
+#include "diff.hpp"
 
 namespace {
 
@@ -65,7 +28,7 @@ using bimpk::kNumOri;
 struct DScale {
     bimph::ScaleGeom g;
     bimpk::CellParams cp;
-    float2* Q = nullptr;   // 8 x FH x FW bank spectra
+    float2* Q = nullptr;   // 8 x FW x FH bank spectra, kx-major
     float* G = nullptr;    // 5 x FW x FH quadrature bank Re(Q_o) / (FH*FW), kx-major
     int Hc = 0, Wc = 0, ldc = 0;  // complex-cell region of the forward (as in detection)
     float2* DT = nullptr;  // forward: (FW/2+1) x FH half spectrum, column-major, per image
@@ -89,20 +52,19 @@ struct bimp_diff {
     std::vector<int> lw, lh;
     std::vector<float*> lev, glev;
     std::map<int, float2*> tw;
-    size_t Pmax = 0;
-    float2 *Dhat = nullptr, *Z = nullptr, *acc = nullptr;
-    float2* Yc = nullptr;  // backward: 8 x kW tap rows of Y_o
-    size_t ycSize = 0;
     // forward: scales of one level and transform size share each launch (first, count)
     std::vector<std::pair<int, int>> groups;
     float2 *R = nullptr, *T = nullptr;  // forward: row spectra and inverse-column output
     float* Sf = nullptr;                // forward: single-stopped maps (scratch)
     size_t rSize = 0, tSize = 0;
-    float *C = nullptr, *Wm = nullptr, *gC = nullptr, *S = nullptr, *taps = nullptr;
+    float* taps = nullptr;              // Ke, Ko of the scale being set up
     unsigned* maxslot = nullptr;
+    // backward: work buffers of up to `entries` (scale, image) pairs per launch
+    bimpk::AdjBuffers adj{};
+    int entries = 1, kwMax = 0;
     float* partials = nullptr;
     int maxBlocks = 0;
-    int nbMax = 1;  // images per backward launch (the per-image buffers hold that many)
+    int nbMax = 8;  // images whose pyramids are held at once
     std::string err;
 };
 
@@ -119,13 +81,6 @@ int dfail(bimp_diff* d, int code, const std::string& m) {
         if (e_ != hipSuccess)                                                           \
             return dfail(d, BIMP_E_DEVICE, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
-
-// In-place 2D complex transform of `nb` FH x FW maps (scratch of the same size).
-int fft2(bimp_diff* d, float2* a, int nb, int FH, int FW, bool inv, hipStream_t s) {
-    DCHK(d, bimpk::diff_rows(a, nb * FH, FW, inv, d->tw[FW], s));
-    DCHK(d, bimpk::diff_cols(a, FH, FW, nb, inv, d->tw[FH], s));
-    return BIMP_OK;
-}
 
 int set_params(bimp_diff* d, float ratio, float gamma, hipStream_t s) {
     for (auto& x : d->sc) {
@@ -148,9 +103,11 @@ int set_params(bimp_diff* d, float ratio, float gamma, hipStream_t s) {
         DCHK(d, hipMemcpy(d->taps, ke.data(), ke.size() * 4, hipMemcpyHostToDevice));
         DCHK(d, hipMemcpy(d->taps + ke.size(), ko.data(), ko.size() * 4, hipMemcpyHostToDevice));
         DCHK(d, hipMemcpy(x.dK, dk.data(), dk.size() * 4, hipMemcpyHostToDevice));
-        DCHK(d, bimpk::diff_bank_pad(d->taps, d->taps + ke.size(), g.kW, g.kX, g.FH, g.FW, x.Q, s));
-        const int st = fft2(d, x.Q, kNumOri, g.FH, g.FW, false, s);
-        if (st) return st;
+        float2* const rows = d->adj.T;  // free here: no pass of this context is under way
+        DCHK(d, bimpk::diff_bank_pad(d->taps, d->taps + ke.size(), g.kW, g.kX, g.FH, g.FW, rows, s));
+        DCHK(d, bimpk::diff_rows(rows, kNumOri * g.FH, g.FW, d->tw[g.FW], s));
+        DCHK(d, bimpk::diff_cols_kx(rows, g.FH, g.FH, g.FW, bimpk::AdjInts{}, 1, kNumOri, x.Q,
+                                    d->tw[g.FH], s));
         DCHK(d, bimpk::diff_q_to_g(x.Q, g.FH, g.FW, 1.0f / ((float)g.FH * (float)g.FW), x.G, s));
         DCHK(d, hipStreamSynchronize(s));
     }
@@ -159,7 +116,6 @@ int set_params(bimp_diff* d, float ratio, float gamma, hipStream_t s) {
     return BIMP_OK;
 }
 
-// Float pyramid of one image into d->lev.
 // Float pyramids of nb consecutive images into d->lev (level l of image b at
 // lev[l] + b * lw[l] * lh[l]).
 int pyramid(bimp_diff* d, const float* img, int nb, hipStream_t s) {
@@ -168,33 +124,6 @@ int pyramid(bimp_diff* d, const float* img, int nb, hipStream_t s) {
     for (int l = 1; l <= d->maxLevel; ++l)
         DCHK(d, bimpk::diff_pyr_down(d->lev[l - 1], d->lw[l - 1], d->lh[l - 1], d->lev[l], d->lw[l],
                                      d->lh[l], nb, s));
-    return BIMP_OK;
-}
-
-// Forward of one scale for the backward pass, for the nb images whose pyramids are in
-// d->lev: Dhat, Z, C per image on the whole FH x FW domain (Z and C valid in rows [0, Hc)),
-// and the D maps into scratch.
-int scale_forward(bimp_diff* d, DScale& x, int nb, hipStream_t s) {
-    const auto& g = x.g;
-    const size_t P = (size_t)g.FH * g.FW;
-    const float sc = 255.0f * d->opt.input_scale;
-    DCHK(d, bimpk::diff_pad(d->lev[g.level], d->lw[g.level],
-                            (size_t)d->lw[g.level] * d->lh[g.level], g.H, g.W, g.FH, g.FW, g.kX,
-                            sc, d->Dhat, nb, s));
-    int st = fft2(d, d->Dhat, nb, g.FH, g.FW, false, s);
-    if (st) return st;
-    DCHK(d, bimpk::diff_spec_mul(d->Dhat, x.Q, d->Z, P, nb, 1.0f / (float)P, s));
-    // inverse: columns first, then only the rows [0, Hc) the cells stencil and its adjoint
-    // read (the rest of Z and C is left column-transformed, finite, and never read)
-    DCHK(d, bimpk::diff_cols(d->Z, g.FH, g.FW, kNumOri * nb, true, d->tw[g.FH], s));
-    DCHK(d, bimpk::diff_rows_maps(d->Z, kNumOri * nb, x.Hc, P, g.FW, true, d->tw[g.FW], s));
-    DCHK(d, bimpk::diff_mag(d->Z, d->C, (size_t)kNumOri * P * nb, s));
-    bimpk::CellScale cs[bimpk::kCellMaxScales];
-    for (int b = 0; b < nb; ++b)
-        cs[b] = bimpk::CellScale{d->C + (size_t)b * kNumOri * P, g.FH, g.FW, g.FH, g.FW, g.H,
-                                 g.W, x.cp, d->S + (size_t)b * 2 * P + P,
-                                 d->S + (size_t)b * 2 * P, d->maxslot};
-    DCHK(d, bimpk::launch_cells(cs, nb, s));
     return BIMP_OK;
 }
 
@@ -252,6 +181,42 @@ int group_forward(bimp_diff* d, int first, int n, int img0, int nb, float* resp,
     return BIMP_OK;
 }
 
+// Backward of scales first..first+n-1 (one level, one transform size) for nb images from img0
+// of the pyramids in d->lev: adds to (with `fresh`: sets) their level gradients in d->glev and
+// writes their parameter partials.  gD: the upstream gradient of image img0's response vector.
+int group_backward(bimp_diff* d, int first, int n, int img0, int nb, const float* gD, bool fresh,
+                   size_t pstride, hipStream_t s) {
+    const DScale& x0 = d->sc[first];
+    const auto& g = x0.g;
+    bimpk::AdjSet set{};
+    set.n = n;
+    for (int j = 0; j < n; ++j) {
+        const DScale& x = d->sc[first + j];
+        set.kX[j] = x.g.kX;
+        set.kW[j] = x.g.kW;
+        set.Q[j] = x.Q;
+        set.dK[j] = x.dK;
+        set.resp[j] = x.respOff;
+        set.cp[j] = x.cp;
+    }
+    const size_t lsz = (size_t)d->lw[g.level] * d->lh[g.level];
+    const bimpk::AdjLevel L{g.H, g.W, g.FH, g.FW, x0.Hc, nb, d->lw[g.level], lsz,
+                            255.0f * d->opt.input_scale,
+                            1.0f / (float)((size_t)g.FH * g.FW), d->lev[g.level] + img0 * lsz};
+    const float2 *twH = d->tw[g.FH], *twW = d->tw[g.FW];
+    const auto& w = d->adj;
+    DCHK(d, bimpk::diff_backward_rows(set, L, w, twW, s));
+    DCHK(d, bimpk::diff_cols_kx(w.T, g.H, g.FH, g.FW, set.ints(set.kX), n, n * nb, w.D, twH, s));
+    DCHK(d, bimpk::diff_z_cols(set, L, w, twH, s));
+    DCHK(d, bimpk::diff_cells_grad(set, L, w, gD, d->respSize, twW, s));
+    DCHK(d, bimpk::diff_adj_cols(set, L, w, d->kwMax, twH, s));
+    DCHK(d, bimpk::diff_adj_rows(set, L, w, d->kwMax, fresh, d->glev[g.level] + img0 * lsz,
+                                 d->lh[g.level],
+                                 d->partials + pstride * img0 + 2 * (size_t)d->maxBlocks * first,
+                                 pstride, 2 * d->maxBlocks, twW, s));
+    return BIMP_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -302,7 +267,6 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
         x.ldc = (x.Wc + 31) / 32 * 32;
 
         d->maxLevel = std::max(d->maxLevel, x.g.level);
-        d->Pmax = std::max(d->Pmax, (size_t)x.g.FH * x.g.FW);
         sizes.push_back(x.g.FH);
         sizes.push_back(x.g.FW);
         d->sc.push_back(x);
@@ -331,16 +295,20 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
         d->lw[l] = (d->lw[l - 1] + 1) / 2;
         d->lh[l] = (d->lh[l - 1] + 1) / 2;
     }
-    // images per backward launch: up to the cells launch's 8 jobs, while the per-image
-    // buffers (8 complex and 44 real maps of the largest transform) stay within 4 GB
-    {
-        size_t pm = 0;
-        for (const auto& x : d->sc) pm = std::max(pm, (size_t)x.g.FH * x.g.FW);
-        const size_t per = pm * (2 * sizeof(float2) + kNumOri * sizeof(float2) +
-                                 (2 + 4) * kNumOri * sizeof(float) + 2 * sizeof(float));
-        d->nbMax = (int)std::max<size_t>(1, std::min<size_t>(bimpk::kCellMaxScales,
-                                                             (size_t(4) << 30) / per));
+    // (scale, image) pairs per backward launch: up to 32, while their buffers (two complex maps
+    // of the padded size, the gradient's pairs and, per orientation, two complex and one real
+    // map) stay within 4 GB.  More pairs mean fewer and longer launches: eight 512 x 512 images
+    // took 2277, 2084 and 2017 us with 8, 16 and 32, five 200 x 130 images 616, 479 and 350 us.
+    size_t pm = 0, kwfw = 0;
+    for (const auto& x : d->sc) {
+        pm = std::max(pm, (size_t)x.g.FH * x.g.FW);
+        kwfw = std::max(kwfw, (size_t)x.g.FW);
+        d->kwMax = std::max(d->kwMax, x.g.kW);
     }
+    const size_t per = pm * (2 * sizeof(float2) + sizeof(uint2) +
+                             kNumOri * (2 * sizeof(float2) + sizeof(float)));
+    d->entries = (int)std::max<size_t>(1, std::min<size_t>(32, (size_t(4) << 30) / per));
+    const size_t NE = (size_t)d->entries;
     const size_t NB = (size_t)d->nbMax;
     d->lev.assign(d->maxLevel + 1, nullptr);
     d->glev.assign(d->maxLevel + 1, nullptr);
@@ -348,12 +316,10 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
         if (hipMalloc(&d->lev[l], NB * d->lw[l] * d->lh[l] * 4) != hipSuccess ||
             hipMalloc(&d->glev[l], NB * d->lw[l] * d->lh[l] * 4) != hipSuccess)
             return bail(BIMP_E_ALLOC);
-    const size_t P = d->Pmax;
     size_t maxTaps = 0;
     for (auto& x : d->sc) {
         const size_t kk = (size_t)x.g.kW * x.g.kW;
         maxTaps = std::max(maxTaps, kk);
-        d->ycSize = std::max(d->ycSize, (size_t)kNumOri * x.g.kW * x.g.FW);
         d->maxBlocks = std::max(d->maxBlocks, bimpk::diff_param_blocks(x.g.kW));
         if (hipMalloc(&x.Q, (size_t)kNumOri * x.g.FH * x.g.FW * sizeof(float2)) != hipSuccess ||
             hipMalloc(&x.G, (size_t)bimpk::kUniqueOri * x.g.FH * x.g.FW * sizeof(float)) != hipSuccess ||
@@ -362,19 +328,19 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
             hipMalloc(&x.dK, 4 * kNumOri * kk * sizeof(float)) != hipSuccess)
             return bail(BIMP_E_ALLOC);
     }
-    if (hipMalloc(&d->Dhat, NB * P * sizeof(float2)) != hipSuccess ||
-        hipMalloc(&d->acc, NB * P * sizeof(float2)) != hipSuccess ||
-        hipMalloc(&d->Z, NB * kNumOri * P * sizeof(float2)) != hipSuccess ||
-        hipMalloc(&d->C, NB * kNumOri * P * sizeof(float)) != hipSuccess ||
-        hipMalloc(&d->gC, NB * kNumOri * P * sizeof(float)) != hipSuccess ||
-        hipMalloc(&d->Wm, NB * 4 * kNumOri * P * sizeof(float)) != hipSuccess ||
-        hipMalloc(&d->S, NB * 2 * P * sizeof(float)) != hipSuccess ||
+    auto& w = d->adj;
+    if (hipMalloc(&w.D, NE * pm * sizeof(float2)) != hipSuccess ||
+        hipMalloc(&w.A, NE * pm * sizeof(float2)) != hipSuccess ||
+        hipMalloc(&w.T, NE * kNumOri * pm * sizeof(float2)) != hipSuccess ||
+        hipMalloc(&w.Z, NE * kNumOri * pm * sizeof(float2)) != hipSuccess ||
+        hipMalloc(&w.C, NE * kNumOri * pm * sizeof(float)) != hipSuccess ||
+        hipMalloc(&w.gm, NE * pm * sizeof(uint2)) != hipSuccess ||
+        hipMalloc(&w.Yc, NE * kNumOri * d->kwMax * kwfw * sizeof(float2)) != hipSuccess ||
         hipMalloc(&d->taps, 2 * kNumOri * maxTaps * sizeof(float)) != hipSuccess ||
         hipMalloc(&d->maxslot, sizeof(unsigned)) != hipSuccess ||
         hipMalloc(&d->R, d->rSize * sizeof(float2)) != hipSuccess ||
         hipMalloc(&d->T, d->tSize * sizeof(float2)) != hipSuccess ||
         hipMalloc(&d->Sf, (size_t)bimpk::kMaxBatch * d->respSize * sizeof(float)) != hipSuccess ||
-        hipMalloc(&d->Yc, NB * d->ycSize * sizeof(float2)) != hipSuccess ||
         hipMalloc(&d->partials, NB * 2 * (size_t)d->maxBlocks * d->sc.size() * sizeof(float)) !=
                 hipSuccess)
         return bail(BIMP_E_ALLOC);
@@ -411,9 +377,9 @@ int bimp_diff_destroy(bimp_diff* d) {
     for (auto* p : d->lev) (void)hipFree(p);
     for (auto* p : d->glev) (void)hipFree(p);
     for (auto& kv : d->tw) (void)hipFree(kv.second);
-    for (void* p : {(void*)d->Dhat, (void*)d->acc, (void*)d->Z, (void*)d->C,
-                    (void*)d->gC, (void*)d->Wm, (void*)d->S, (void*)d->taps, (void*)d->maxslot,
-                    (void*)d->partials, (void*)d->R, (void*)d->T, (void*)d->Sf, (void*)d->Yc})
+    for (void* p : {(void*)d->adj.D, (void*)d->adj.A, (void*)d->adj.T, (void*)d->adj.Z,
+                    (void*)d->adj.C, (void*)d->adj.gm, (void*)d->adj.Yc, (void*)d->taps,
+                    (void*)d->maxslot, (void*)d->partials, (void*)d->R, (void*)d->T, (void*)d->Sf})
         (void)hipFree(p);
     delete d;
     return BIMP_OK;
@@ -453,45 +419,34 @@ int bimp_diff_backward(bimp_diff* d, const float* d_img, int nimg, const float* 
     if (!d || !d_img || !d_grad_resp || !d_grad_img || nimg <= 0) return BIMP_E_ARG;
     hipStream_t s = (hipStream_t)stream;
     const size_t isz = (size_t)d->width * d->height;
-    const float sc = 255.0f * d->opt.input_scale;
     double gr = 0, gg = 0;
     std::vector<float> part;
     const size_t pstride = 2 * (size_t)d->maxBlocks * d->sc.size();  // partials per image
-    // chunks of up to nbMax images: every launch below covers the chunk's images at once
+    // chunks of images whose pyramids are held; each group then takes as many (scale, image)
+    // pairs per launch as the work buffers hold
     for (int b0 = 0; b0 < nimg; b0 += d->nbMax) {
         const int nb = std::min(d->nbMax, nimg - b0);
         int st = pyramid(d, d_img + b0 * isz, nb, s);
         if (st) return st;
-        for (int l = 0; l <= d->maxLevel; ++l)
-            DCHK(d, bimpk::diff_fill(d->glev[l], (size_t)nb * d->lw[l] * d->lh[l], s));
-        for (size_t si = 0; si < d->sc.size(); ++si) {
-            DScale& x = d->sc[si];
-            const auto& g = x.g;
-            const size_t P = (size_t)g.FH * g.FW;
-            const float invN = 1.0f / (float)P;
-            // recompute the responses (the D maps go to scratch)
-            if ((st = scale_forward(d, x, nb, s))) return st;
-            DCHK(d, bimpk::diff_cells_adj(d->C, g.FH, g.FW, g.H, g.W, x.cp,
-                                          d_grad_resp + b0 * d->respSize + x.respOff, d->respSize,
-                                          d->Wm, d->gC, nb, s));
-            DCHK(d, bimpk::diff_grad_z(d->gC, d->Z, (size_t)kNumOri * P * nb, s));
-            // gZ is zero outside rows [0, Hc): their row transforms are zero, not computed
-            DCHK(d, bimpk::diff_rows_maps(d->Z, kNumOri * nb, x.Hc, P, g.FW, false, d->tw[g.FW], s));
-            DCHK(d, bimpk::diff_cols(d->Z, g.FH, g.FW, kNumOri * nb, false, d->tw[g.FH], s));
-            DCHK(d, bimpk::diff_accum_conjq(x.Q, d->Z, d->acc, P, nb, invN, s));
-            if ((st = fft2(d, d->acc, nb, g.FH, g.FW, true, s))) return st;
-            DCHK(d, bimpk::diff_pad_adj(d->acc, g.H, g.W, g.FH, g.FW, g.kX, sc, d->glev[g.level],
-                                        d->lw[g.level], (size_t)d->lw[g.level] * d->lh[g.level],
-                                        nb, s));
-            DCHK(d, bimpk::diff_mul_conjd(d->Z, d->Dhat, P, nb, invN, s));
-            // Y_o = IFFT2(...) is read at the kW x kW taps only: columns, then the kW tap rows
-            DCHK(d, bimpk::diff_cols(d->Z, g.FH, g.FW, kNumOri * nb, true, d->tw[g.FH], s));
-            DCHK(d, bimpk::diff_gather_tap_rows(d->Z, g.kW, g.kX, g.FH, g.FW, d->Yc, nb, s));
-            DCHK(d, bimpk::diff_rows(d->Yc, kNumOri * g.kW * nb, g.FW, true, d->tw[g.FW], s));
-            DCHK(d, bimpk::diff_param_partials(d->Yc, g.kW, g.kX, g.FW, x.dK,
-                                               d->partials + 2 * (size_t)d->maxBlocks * si,
-                                               pstride, nb, s));
+        std::vector<char> fresh(d->maxLevel + 1, 1);
+        for (const auto& gr : d->groups) {
+            // (a group holds at most kMaxBatch scales)
+            for (int j0 = 0; j0 < gr.second; j0 += d->entries) {
+                const int n = std::min(gr.second - j0, d->entries);
+                const int nbg = std::max(1, d->entries / n);
+                const int level = d->sc[gr.first].g.level;
+                for (int b = 0; b < nb; b += nbg)
+                    if ((st = group_backward(d, gr.first + j0, n, b, std::min(nbg, nb - b),
+                                             d_grad_resp + (size_t)(b0 + b) * d->respSize,
+                                             fresh[level] != 0, pstride, s)))
+                        return st;
+                fresh[level] = 0;
+            }
         }
+        // (a level no scale uses starts at zero as well)
+        for (int l = 0; l <= d->maxLevel; ++l)
+            if (fresh[l])
+                DCHK(d, bimpk::diff_fill(d->glev[l], (size_t)nb * d->lw[l] * d->lh[l], s));
         for (int l = d->maxLevel; l >= 1; --l)
             DCHK(d, bimpk::diff_pyr_down_adj(d->glev[l], d->lw[l], d->lh[l], d->glev[l - 1],
                                              d->lw[l - 1], d->lh[l - 1], nb, s));

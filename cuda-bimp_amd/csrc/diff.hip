@@ -11,12 +11,17 @@
 //   gPd  = Re IFFT(sum_o conj(Qhat_o) * Ghat_o) / N,
 //   Y_o  = IFFT(Ghat_o * conj(FFT(Pd))) / N = dL/dKe_o + i dL/dKo_o at the tap positions,
 //   then gL = s * pad^T(gPd) and the float-pyramid adjoint down to the image.
-// All transforms are full complex 2D FFTs: batched row transforms, then column transforms
-// staged through LDS.
+// All transforms are full complex 2D FFTs.  The backward keeps spectra kx-major (a column's FH
+// values contiguous), so that column transforms read D and Q straight into registers, and what
+// passes between row and column transforms in blocks of kb columns (kb * rows contiguous).
+// Everything elementwise rides in a transform's load or store: eight launches per group of
+// scales and images (k_pad_rows .. k_img_rows), besides the tap rows and their sums.
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
+#include "diff.hpp"
 #include "fft_device.hpp"
-#include "kernels.hpp"
 
 namespace bimpk {
 
@@ -28,22 +33,26 @@ using bimpdev::out_index;
 
 constexpr int kRowThreads = 256;
 
-// Batched in-place complex transforms of rows of length N: `rows` rows in all, the first
-// `per_map` rows of each map of `map_stride` elements (per_map = rows: contiguous rows).
+// A thread's group of TPV lanes in its workgroup: one wavefront or two share it from 64 lanes
+// on, so it (and every row index and pointer made from it) stays in scalar registers there.
+template <int TPV>
+__device__ __forceinline__ int group_of(int tid) {
+    return TPV >= 64 ? __builtin_amdgcn_readfirstlane(tid / TPV) : tid / TPV;
+}
+
+// In-place complex transforms of `rows` contiguous rows of length N.
 template <int N, bool INV>
 __global__ void __launch_bounds__(kRowThreads) k_c2c_rows(float2* __restrict__ data, int rows,
-                                                          int per_map, size_t map_stride,
                                                           const float2* __restrict__ tw) {
     using C = FFTCfg<N>;
     constexpr int GPB = kRowThreads / C::TPV;
     extern __shared__ float lds[];
-    const int grp = threadIdx.x / C::TPV, lane = threadIdx.x % C::TPV;
+    const int grp = group_of<C::TPV>(threadIdx.x), lane = threadIdx.x % C::TPV;
     // every group transforms (a spare one row 0, unstored): a 128-lane group's stages take
     // the workgroup barrier
     const int row = blockIdx.x * GPB + grp;
     const bool act = row < rows;
-    const int r = act ? row : 0;
-    float2* p = data + (size_t)(r / per_map) * map_stride + (size_t)(r % per_map) * N;
+    float2* p = data + (size_t)(act ? row : 0) * N;
     float2 v[C::E];
 #pragma unroll
     for (int e = 0; e < C::E; ++e) v[e] = p[in_index<N>(e, lane)];
@@ -54,46 +63,49 @@ __global__ void __launch_bounds__(kRowThreads) k_c2c_rows(float2* __restrict__ d
     }
 }
 
-// In-place complex transforms of the columns of `nb` N x W maps ([b][r][c], r < N): a
-// workgroup stages CB adjacent columns through LDS (each row contributes CB contiguous
-// values), one group of lanes transforms each column, and the results leave the same way.
-// It replaces transpose + row transforms + transpose and moves each value once each way.
+// Column kernels: a workgroup owns CB adjacent columns, one group of TPV lanes each; a column
+// stages through LDS with stride S (2 (mod 16) complex spreads the staging accesses).
 template <int N>
-struct CColCfg {
-    static constexpr int TPV = FFTCfg<N>::TPV;
-    static constexpr int CB = TPV == 64 ? (N <= 2048 ? 8 : 4) : (512 / TPV > 16 ? 16 : 512 / TPV);
+struct ACfg {
+    static constexpr int TPV = FFTCfg<N>::TPV, E = FFTCfg<N>::E;
+    static constexpr int CB = diff_block_columns(N);
     static constexpr int THREADS = CB * TPV;
-    static constexpr int S = N + 2;  // column stride (complex): 2 (mod 16) spreads the staging
+    static constexpr int S = N + 2;
+    static constexpr int LDS = CB * S * (int)sizeof(float2);
 };
 
-template <int N, bool INV>
-__global__ void __launch_bounds__(CColCfg<N>::THREADS) k_c2c_cols(float2* __restrict__ data,
-                                                                   int W,
-                                                                   const float2* __restrict__ tw) {
-    using C = FFTCfg<N>;
-    using CC = CColCfg<N>;
+// Columns of `maps` row-major maps of H x W into kx-major spectra of FH x W: row y of the
+// transform reads row y of the map, rows [H, H+k) its last row and later ones row 0 (the clamp
+// padding).  One entry of `k` per scale of the group.
+template <int N>
+__global__ void __launch_bounds__(ACfg<N>::THREADS) k_cols_kx(const float2* __restrict__ in, int H,
+                                                               int W, AdjInts k, int nscales,
+                                                               float2* __restrict__ out,
+                                                               const float2* __restrict__ tw) {
+    using A = ACfg<N>;
     extern __shared__ float2 lds2[];
-    float2* map = data + (size_t)blockIdx.y * N * W;
-    const int c0 = blockIdx.x * CC::CB;
-    for (int t = threadIdx.x; t < N * CC::CB; t += CC::THREADS) {
-        const int b = t % CC::CB, r = t / CC::CB;
-        lds2[b * CC::S + r] = c0 + b < W ? map[(size_t)r * W + c0 + b] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    const int g = threadIdx.x / C::TPV, lane = threadIdx.x % C::TPV;
-    float2* my = lds2 + (size_t)g * CC::S;
-    float2 v[C::E];
+    const int map = blockIdx.y, kX = k.v[map % nscales];
+    const float2* src = in + (size_t)map * H * W;
+    const int c0 = blockIdx.x * A::CB, b = threadIdx.x % A::CB, y0 = threadIdx.x / A::CB;
+    float2 v[A::E];
 #pragma unroll
-    for (int e = 0; e < C::E; ++e) v[e] = my[in_index<N>(e, lane)];
-    bimpdev::stage_sync<C::TPV>();
-    bimpdev::fft<N, INV>(v, reinterpret_cast<float*>(my), lane, tw);
-#pragma unroll
-    for (int e = 0; e < C::E; ++e) my[out_index<N>(e, lane)] = v[e];
-    __syncthreads();
-    for (int t = threadIdx.x; t < N * CC::CB; t += CC::THREADS) {
-        const int b = t % CC::CB, r = t / CC::CB;
-        if (c0 + b < W) map[(size_t)r * W + c0 + b] = lds2[b * CC::S + r];
+    for (int i = 0; i < A::E; ++i) {
+        const int y = y0 + i * A::TPV;
+        const int ry = y < H ? y : (y < H + kX ? H - 1 : 0);
+        v[i] = src[(size_t)ry * W + c0 + b];
     }
+#pragma unroll
+    for (int i = 0; i < A::E; ++i) lds2[b * A::S + y0 + i * A::TPV] = v[i];
+    __syncthreads();
+    const int g = group_of<A::TPV>(threadIdx.x), lane = threadIdx.x % A::TPV;
+    float2* my = lds2 + (size_t)g * A::S;
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) v[e] = my[in_index<N>(e, lane)];
+    bimpdev::stage_sync<A::TPV>();
+    bimpdev::fft<N, false>(v, reinterpret_cast<float*>(my), lane, tw);
+    float2* dst = out + ((size_t)map * W + c0 + g) * N;
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) dst[out_index<N>(e, lane)] = v[e];
 }
 
 __device__ __forceinline__ int reflect101(int t, int n) {
@@ -166,74 +178,12 @@ __global__ void k_pyr_down_adj(const float* __restrict__ gdst, int dw, int dh,
     gsrc[(size_t)y * sw + x] += acc;
 }
 
-__device__ __forceinline__ int clamp_src(int y, int H, int k) { return y < H ? y : (y < H + k ? H - 1 : 0); }
-
-// Pd = s * pad(L) as complex (imaginary part 0).  L is the top-left H x W region of a level
-// image with `pitch` floats per row (a level is (n+1)/2 wide, its data n/2).
-// blockIdx.z: image of the batch (level images lstride floats apart, outputs FH*FW apart)
-__global__ void k_pad_fwd(const float* __restrict__ L, int pitch, size_t lstride, int H, int W,
-                          int FH, int FW, int k, float s, float2* __restrict__ out) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-    if (x >= FW) return;
-    L += blockIdx.z * lstride;
-    out += (size_t)blockIdx.z * FH * FW;
-    out[(size_t)y * FW + x] =
-            make_float2(s * L[(size_t)clamp_src(y, H, k) * pitch + clamp_src(x, W, k)], 0.f);
-}
-
-// Source rows of the padded image that read data row r: r itself, the band [H, H+k) for
-// r = H-1 and the band [H+k, F) for r = 0.
-__device__ __forceinline__ void pad_band(int r, int H, int F, int k, int* lo1, int* hi1) {
-    *lo1 = 0;
-    *hi1 = 0;
-    if (r == H - 1) {
-        *lo1 = H;
-        *hi1 = min(H + k, F);
-    } else if (r == 0) {
-        *lo1 = min(H + k, F);
-        *hi1 = F;
-    }
-}
-
-// gL += s * pad^T(Re gPd) over the top-left H x W region of gL (`pitch` floats per row)
-__global__ void k_pad_adj(const float2* __restrict__ g, int H, int W, int FH, int FW, int k,
-                          float s, float* __restrict__ gL, int pitch, size_t lstride) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-    if (x >= W) return;
-    g += (size_t)blockIdx.z * FH * FW;
-    gL += blockIdx.z * lstride;
-    int ylo, yhi, xlo, xhi;
-    pad_band(y, H, FH, k, &ylo, &yhi);
-    pad_band(x, W, FW, k, &xlo, &xhi);
-    float acc = 0.f;
-    for (int yy = -1; yy < yhi - ylo; ++yy) {
-        const int sy = yy < 0 ? y : ylo + yy;
-        const float2* row = g + (size_t)sy * FW;
-        acc += row[x].x;
-        for (int xx = xlo; xx < xhi; ++xx) acc += row[xx].x;
-    }
-    gL[(size_t)y * pitch + x] += s * acc;
-}
-
-// G_o(ky, kx) = Re Q_o(ky, kx) / (FH*FW) for o = 0..4, stored kx-major (G[o][kx][ky]): the
-// quadrature bank layout of the detection path's inverse column pass, from the spectra Q of
-// the current parameters.  32 x 32 tiles transposed through LDS.
-__global__ void __launch_bounds__(256) k_q_to_g(const float2* __restrict__ Q, int FH, int FW,
-                                               float invN, float* __restrict__ G) {
-    __shared__ float tile[32][33];
-    const int o = blockIdx.z, kx0 = blockIdx.x * 32, ky0 = blockIdx.y * 32;
-    const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
-    const float2* q = Q + (size_t)o * FH * FW;
-    for (int r = ty; r < 32; r += 8) {
-        const int ky = ky0 + r, kx = kx0 + tx;
-        if (ky < FH && kx < FW) tile[r][tx] = q[(size_t)ky * FW + kx].x * invN;
-    }
-    __syncthreads();
-    float* g = G + (size_t)o * FW * FH;
-    for (int r = ty; r < 32; r += 8) {
-        const int kx = kx0 + r, ky = ky0 + tx;
-        if (ky < FH && kx < FW) g[(size_t)kx * FH + ky] = tile[tx][r];
-    }
+// G_o(ky, kx) = Re Q_o(ky, kx) / (FH*FW) for o = 0..4, kx-major like Q: the quadrature bank of
+// the detection path's inverse column pass, from the spectra Q of the current parameters.
+__global__ void k_q_to_g(const float2* __restrict__ Q, size_t n, float invN,
+                         float* __restrict__ G) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) G[i] = Q[i].x * invN;
 }
 
 // Padded complex kernels of the 8 orientations: tap (r, c) sits at ((r-kX) mod FH,
@@ -251,35 +201,136 @@ __global__ void k_bank_pad(const float* __restrict__ ke, const float* __restrict
     out[((size_t)o * FH + y) * FW + x] = v;
 }
 
-// Z_o = D * Q_o * invN for the 8 orientations; nb images (D: nb maps of n, Z: nb x 8 maps).
-__global__ void k_spec_mul(const float2* __restrict__ D, const float2* __restrict__ Q,
-                           float2* __restrict__ Z, size_t n, int nb, float invN) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * nb) return;
-    const size_t b = t / n, i = t - b * n;
-    const float2 d = D[t];
-    float2* z = Z + b * kNumOri * n;
+// ---------------------------------------------------------------- backward pipeline
+// The launches below cover the entries of a group, scales of one level and transform size by
+// images: entry k = image * nscales + scale (AdjSet), each with its own buffers.
+
+// A product that rounds once: the compiler must not contract it into the additions that the
+// following transform starts with, so that a value is the same wherever it is computed.
+__device__ __forceinline__ float mul1(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+__device__ __forceinline__ float2 scale1(float2 a, float s) {
+    return make_float2(mul1(a.x, s), mul1(a.y, s));
+}
+// |z|^2, in the same operations everywhere
+__device__ __forceinline__ float norm1(float2 z) { return fmaf(z.x, z.x, mul1(z.y, z.y)); }
+
+__device__ __forceinline__ int clamp_src(int y, int H, int k) { return y < H ? y : (y < H + k ? H - 1 : 0); }
+
+// Row transforms of the padded image's distinct rows y < H: Pd = s * pad(L) as complex, L the
+// top-left H x W region of a level image (`pitch` floats per row, images lstride apart).
+template <int N>
+__global__ void __launch_bounds__(kRowThreads) k_pad_rows(const float* __restrict__ L, int pitch,
+                                                          size_t lstride, int H, int W, AdjInts k,
+                                                          int nscales, float s, int rows,
+                                                          float2* __restrict__ out,
+                                                          const float2* __restrict__ tw) {
+    using C = FFTCfg<N>;
+    constexpr int GPB = kRowThreads / C::TPV;
+    extern __shared__ float lds[];
+    const int grp = group_of<C::TPV>(threadIdx.x), lane = threadIdx.x % C::TPV;
+    // every group transforms (a spare one row 0, unstored): a 128-lane group's stages take
+    // the workgroup barrier
+    const int row = blockIdx.x * GPB + grp;
+    const bool act = row < rows;
+    const int r = act ? row : 0, entry = r / H, y = r % H;
+    const int kX = k.v[entry % nscales];
+    const float* src = L + (entry / nscales) * lstride + (size_t)y * pitch;
+    float zero = 0.f;
+    asm volatile("" : "+v"(zero));  // a runtime zero: the transform's arithmetic stays general
+    float2 v[C::E];
 #pragma unroll
-    for (int o = 0; o < kNumOri; ++o) {
-        const float2 q = Q[(size_t)o * n + i];
-        z[(size_t)o * n + i] =
-            make_float2((d.x * q.x - d.y * q.y) * invN, (d.x * q.y + d.y * q.x) * invN);
+    for (int e = 0; e < C::E; ++e)
+        v[e] = make_float2(mul1(s, src[clamp_src(in_index<N>(e, lane), W, kX)]), zero);
+    bimpdev::fft<N, false>(v, lds + grp * bimpdev::fft_lds_floats<N>(), lane, tw);
+    if (act) {
+        float2* p = out + (size_t)row * N;
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) p[out_index<N>(e, lane)] = v[e];
     }
 }
 
-__global__ void k_mag(const float2* __restrict__ Z, float* __restrict__ C, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float2 z = Z[i];
-    C[i] = sqrtf(z.x * z.x + z.y * z.y);
+// Z_o's columns: inverse column transforms of D * Q_o / (FH*FW), rows y < Hc into the block
+// layout of T.  Workgroups are dealt round-robin to the eight XCDs; the numbering gives each
+// XCD every eighth column block, its eight orientations back to back (D's columns from L2 after
+// the first), then the images of one scale (that XCD's share of Q stays in its L2), then the
+// scales: 208 us for 32 entries of 512 x 512, 224 us with each orientation on one XCD.
+template <int N>
+__global__ void __launch_bounds__(ACfg<N>::THREADS) k_z_cols(const float2* __restrict__ D,
+                                                             AdjSet set, int nb, int W, int Hc,
+                                                             float invN, float2* __restrict__ T,
+                                                             const float2* __restrict__ tw) {
+    using A = ACfg<N>;
+    extern __shared__ float2 lds2[];
+    const int nblk = W / A::CB, per = (nblk + 7) / 8;
+    int i = blockIdx.x / 8;
+    const int o = i % kNumOri;
+    i /= kNumOri;
+    const int blk = (i % per) * 8 + blockIdx.x % 8;
+    i /= per;
+    if (blk >= nblk) return;  // uniform
+    const int entry = (i % nb) * set.n + i / nb;
+    const int g = group_of<A::TPV>(threadIdx.x), lane = threadIdx.x % A::TPV;
+    const int kx = blk * A::CB + g;
+    const float2* d = D + ((size_t)entry * W + kx) * N;
+    const float2* q = set.Q[entry % set.n] + ((size_t)o * W + kx) * N;
+    float2 v[A::E];
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) {
+        const int i = in_index<N>(e, lane);
+        const float2 dv = d[i], qv = q[i];
+        v[e] = scale1(make_float2(fmaf(dv.x, qv.x, -mul1(dv.y, qv.y)),
+                                  fmaf(dv.y, qv.x, mul1(dv.x, qv.y))), invN);
+    }
+    float2* my = lds2 + (size_t)g * A::S;
+    bimpdev::fft<N, true>(v, reinterpret_cast<float*>(my), lane, tw);
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) my[out_index<N>(e, lane)] = v[e];
+    __syncthreads();
+    float2* t = T + (((size_t)entry * kNumOri + o) * W + (size_t)blk * A::CB) * Hc;
+    const int b = threadIdx.x % A::CB, y0 = threadIdx.x / A::CB;
+#pragma unroll
+    for (int i = 0; i < A::E; ++i) {
+        const int y = y0 + i * A::TPV;
+        if (y < Hc) t[(size_t)y * A::CB + b] = lds2[b * A::S + y];
+    }
 }
 
-// Complex-cell map read with the reference's linear index y*FW + x over the FH x FW array,
-// wrapping past the end (the forward stencil's semantics).
-__device__ __forceinline__ float cat(const float* C, int o, long idx, long P) {
-    if (idx >= P) idx -= P;
-    if (idx < 0) idx += P;
-    return C[(size_t)o * P + idx];
+// Element x of row y in the block layout with kb = 2^sh columns per block.
+__device__ __forceinline__ size_t blk_at(int x, int y, int rows, int sh) {
+    return ((size_t)(x >> sh) * rows + y) << sh | (x & ((1 << sh) - 1));
+}
+
+// Inverse row transforms of T's rows: Z (row-major) and C = |Z|.
+template <int N>
+__global__ void __launch_bounds__(kRowThreads) k_z_rows(const float2* __restrict__ T, int Hc,
+                                                        int sh, int rows, float2* __restrict__ Z,
+                                                        float* __restrict__ Cm,
+                                                        const float2* __restrict__ tw) {
+    using C = FFTCfg<N>;
+    constexpr int GPB = kRowThreads / C::TPV;
+    extern __shared__ float lds[];
+    const int grp = group_of<C::TPV>(threadIdx.x), lane = threadIdx.x % C::TPV;
+    const int row = blockIdx.x * GPB + grp;
+    const bool act = row < rows;
+    const int r = act ? row : 0, map = r / Hc, y = r % Hc;
+    const float2* t = T + (size_t)map * Hc * N;
+    float2 v[C::E];
+#pragma unroll
+    for (int e = 0; e < C::E; ++e) v[e] = t[blk_at(in_index<N>(e, lane), y, Hc, sh)];
+    bimpdev::fft<N, true>(v, lds + grp * bimpdev::fft_lds_floats<N>(), lane, tw);
+    if (act) {
+        float2* z = Z + (size_t)row * N;
+        float* c = Cm + (size_t)row * N;
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) {
+            const int x = out_index<N>(e, lane);
+            z[x] = v[e];
+            c[x] = sqrtf(norm1(v[e]));
+        }
+    }
 }
 
 __device__ __forceinline__ bool valid(int x, int y, int a, int b, int W, int H) {
@@ -287,161 +338,421 @@ __device__ __forceinline__ bool valid(int x, int y, int a, int b, int W, int H) 
     return 2 * bb <= x && x <= W - 2 * bb && 2 * aa <= y && y <= H - 2 * aa;
 }
 
-// Pass 1 of the stencil adjoint: per pixel and orientation, upstream gradient times the
-// active-branch masks of the forward (cuda_bimp.cuh:436-502):
-//   Wd = g [ds > 0], Wt = g [tangential > 0], W1 = g [v2 > 0][v1 > 0], W2 = g [v2 > 0]
-// stored as 4 x 8 maps over the FH x FW grid (zero outside the data region).
-// blockIdx.z: image of the batch (C: 8 maps, Wm: 32 maps per image; gD gstride apart)
-__global__ void k_cells_adj_w(const float* __restrict__ C, int FH, int FW, int H, int W,
-                              CellParams p, const float* __restrict__ gD, size_t gstride,
-                              float* __restrict__ Wm) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
+// Pass 1 of the stencil adjoint: per pixel and orientation, which branches of the forward
+// (cuda_bimp.cuh:436-502) are active where the upstream gradient g is nonzero:
+//   bit o: ds > 0, bit 8 + o: tangential > 0, bit 16 + o: v2 > 0 and v1 > 0, bit 24 + o: v2 > 0
+// stored with g as one 8-byte pair per pixel of H x FW (zero right of the data).  Four
+// float masks per pixel and orientation took 16 times the bytes: 92 us to write and 96 us to
+// gather from per scale of eight 512 x 512 images, against 55 us here.  blockIdx.z: entry.
+__global__ void __launch_bounds__(256) k_branch_bits(const float* __restrict__ C, int Hc, int FH,
+                                                     int FW, int H, int W, AdjSet set,
+                                                     const float* __restrict__ gD, size_t gstride,
+                                                     uint2* __restrict__ out) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, entry = blockIdx.z;
     if (x >= FW) return;
-    const long P = (long)FH * FW, g0 = (long)y * FW + x;
-    C += (size_t)blockIdx.z * kNumOri * P;
-    gD += blockIdx.z * gstride;
-    Wm += (size_t)blockIdx.z * 4 * kNumOri * P;
-    const float g = (y < H && x < W) ? gD[(size_t)y * W + x] : 0.f;
+    const int j = entry % set.n;
+    const CellParams& p = set.cp[j];
+    // complex-cell maps are read with the reference's linear index y*FW + x over the FH x FW
+    // array, wrapping past the end (the forward stencil's semantics); they hold Hc rows, which
+    // is all that valid pixels reach
+    const int P = FH * FW, g0 = y * FW + x;
+    const size_t mp = (size_t)Hc * FW;
+    C += (size_t)entry * kNumOri * mp;
+    gD += (size_t)(entry / set.n) * gstride + set.resp[j];
+    auto cat = [&](const float* m, int idx) {
+        if (idx >= P) idx -= P;
+        if (idx < 0) idx += P;
+        return m[(unsigned)idx];
+    };
+    const float g = x < W ? gD[(size_t)y * W + x] : 0.f;
+    unsigned bits = 0;
+    if (g != 0.f) {
 #pragma unroll
-    for (int o = 0; o < kNumOri; ++o) {
-        float wd = 0.f, wt = 0.f, w1 = 0.f, w2 = 0.f;
-        if (g != 0.f) {
+        for (int o = 0; o < kNumOri; ++o) {
+            const float* Co = C + o * mp;
+            const float* C2 = C + ((o + kNumOri / 2) % kNumOri) * mp;
+            const float c = Co[(unsigned)g0];
             const int a = p.ea[o], b = p.eb[o];
             if (valid(x, y, a, b, W, H)) {
-                const float v = (float)((double)cat(C, o, g0, P) -
-                                        0.5 * (double)cat(C, o, g0 - 2L * a * FW + 2 * b, P) -
-                                        0.5 * (double)cat(C, o, g0 + 2L * a * FW - 2 * b, P));
-                if (v > 0.f) wd = g;
+                const int d1 = 2 * b - 2 * a * FW;
+                const float v = (float)((double)c - 0.5 * (double)cat(Co, g0 + d1) -
+                                        0.5 * (double)cat(Co, g0 - d1));
+                if (v > 0.f) bits |= 1u << o;
             }
             const int ia = p.ia[o], ib = p.ib[o];
             if (valid(x, y, ia, ib, W, H)) {
-                const int o2 = (o + kNumOri / 2) % kNumOri;
-                const float c = cat(C, o, g0, P);
-                const float vt = cat(C, o, g0 - (long)ia * FW - ib, P) - c;
-                if (vt > 0.f) wt = g;
-                const long rr = (long)p.ra[o] * FW + p.rb[o];
-                float v1 = c - 16.f * cat(C, o2, g0 + rr, P);
+                const float vt = cat(Co, g0 - ia * FW - ib) - c;
+                if (vt > 0.f) bits |= 1u << (8 + o);
+                const int rr = p.ra[o] * FW + p.rb[o];
+                float v1 = c - 16.f * cat(C2, g0 + rr);
                 const bool m1 = v1 > 0.f;
                 v1 = m1 ? v1 : 0.f;
-                const float v2 = v1 + c - 16.f * cat(C, o2, g0 - rr, P);
-                if (v2 > 0.f) {
-                    w2 = g;
-                    w1 = m1 ? g : 0.f;
-                }
+                const float v2 = v1 + c - 16.f * cat(C2, g0 - rr);
+                if (v2 > 0.f) bits |= (1u << (24 + o)) | (m1 ? 1u << (16 + o) : 0u);
             }
         }
-        Wm[((size_t)0 * kNumOri + o) * P + g0] = wd;
-        Wm[((size_t)1 * kNumOri + o) * P + g0] = wt;
-        Wm[((size_t)2 * kNumOri + o) * P + g0] = w1;
-        Wm[((size_t)3 * kNumOri + o) * P + g0] = w2;
     }
+    out[(size_t)entry * H * FW + g0] = make_uint2(__float_as_uint(g), bits);
 }
 
-// Pass 2: gather, for each map position p and orientation o, every forward read of C_o(p):
+// Pass 2, in the load of gZ's row transforms: gathers, for a map position q and orientation o,
+// every forward read of C_o(q):
 //   D = sum_o relu(C(x) - C(x+d1)/2 - C(x+d2)/2) - sum_o [relu(C(x+t) - C(x)) + R_o(x)],
-//   R_o(x) = relu(relu(C_o(x) - 16 C_o'(x+r)) + C_o(x) - 16 C_o'(x-r)), o' = o+4.
-// blockIdx.z = image * 8 + orientation
-__global__ void k_cells_adj_g(const float* __restrict__ Wm, int FH, int FW, CellParams p,
-                              float* __restrict__ gC) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-    const int o = blockIdx.z % kNumOri, img = blockIdx.z / kNumOri;
-    if (x >= FW) return;
-    const long P = (long)FH * FW, q = (long)y * FW + x;
-    Wm += (size_t)img * 4 * kNumOri * P;
-    gC += (size_t)img * kNumOri * P;
-    const float* Wd = Wm + ((size_t)0 * kNumOri + o) * P;
-    const float* Wt = Wm + ((size_t)1 * kNumOri + o) * P;
-    const int a = p.ea[o], b = p.eb[o];
-    const long d1 = -2L * a * FW + 2 * b;
-    float acc = cat(Wd, 0, q, P) - 0.5f * cat(Wd, 0, q - d1, P) - 0.5f * cat(Wd, 0, q + d1, P);
-    const long t = -(long)p.ia[o] * FW - p.ib[o];
-    acc += cat(Wt, 0, q, P) - cat(Wt, 0, q - t, P);
-    // own radial term (centre)
-    const float* W1 = Wm + ((size_t)2 * kNumOri + o) * P;
-    const float* W2 = Wm + ((size_t)3 * kNumOri + o) * P;
-    acc -= cat(W1, 0, q, P) + cat(W2, 0, q, P);
+//   R_o(x) = relu(relu(C_o(x) - 16 C_o'(x+r)) + C_o(x) - 16 C_o'(x-r)), o' = o+4,
+// then gZ = gC * Z / |Z| (zero where |Z| = 0) and the forward row transform into T's layout.
+// Bound by HBM (Z in, T out: 212 us at the copy rate for four scales of eight 512 x 512 images);
+// takes 409 us, of which the gather is 165.
+struct Gather {
+    const uint2* gm;  // (g, branch bits), H rows of FW
+    int P, HF;        // FH*FW, H*FW
+    template <bool CHECK>
+    __device__ __forceinline__ uint2 at(int idx) const {
+        if (!CHECK) return gm[(unsigned)idx];
+        if (idx >= P) idx -= P;
+        if (idx < 0) idx += P;
+        return idx < HF ? gm[(unsigned)idx] : make_uint2(0u, 0u);
+    }
+};
+__device__ __forceinline__ float pick(uint2 v, int bit) {
+    return (v.y >> bit) & 1u ? __uint_as_float(v.x) : 0.f;
+}
+struct Taps {
+    int d1, t, rr, o, op;
+};
+template <bool CHECK>
+__device__ __forceinline__ float gather_gc(const Gather& m, const Taps& k, int q) {
+    const uint2 c = m.at<CHECK>(q);
+    float acc = pick(c, k.o) - 0.5f * pick(m.at<CHECK>(q - k.d1), k.o) -
+                0.5f * pick(m.at<CHECK>(q + k.d1), k.o);
+    acc += pick(c, 8 + k.o) - pick(m.at<CHECK>(q - k.t), 8 + k.o);
+    acc -= pick(c, 16 + k.o) + pick(c, 24 + k.o);
     // partner terms: C_o is the second map of orientation o' = o + 4 (mod 8)
-    const int op = (o + kNumOri / 2) % kNumOri;
-    const float* W1p = Wm + ((size_t)2 * kNumOri + op) * P;
-    const float* W2p = Wm + ((size_t)3 * kNumOri + op) * P;
-    const long rr = (long)p.ra[op] * FW + p.rb[op];
-    acc += 16.f * cat(W1p, 0, q - rr, P) + 16.f * cat(W2p, 0, q + rr, P);
-    gC[(size_t)o * P + q] = acc;
+    acc += 16.f * pick(m.at<CHECK>(q - k.rr), 16 + k.op) +
+           16.f * pick(m.at<CHECK>(q + k.rr), 24 + k.op);
+    return acc;
 }
 
-// gZ = gC * Z / |Z| in place over Z (zero where |Z| = 0).
-__global__ void k_grad_z(const float* __restrict__ gC, float2* __restrict__ Z, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float2 z = Z[i];
-    const float m = sqrtf(z.x * z.x + z.y * z.y);
-    const float s = m > 0.f ? gC[i] / m : 0.f;
-    Z[i] = make_float2(z.x * s, z.y * s);
-}
-
-// out = invN * sum_o conj(Q_o) * G_o per image (G: nb x 8 maps of n, out: nb maps)
-__global__ void k_accum_conjq(const float2* __restrict__ Q, const float2* __restrict__ G,
-                              float2* __restrict__ out, size_t n, int nb, float invN) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * nb) return;
-    const size_t b = t / n, i = t - b * n;
-    const float2* gb = G + b * kNumOri * n;
-    float re = 0.f, im = 0.f;
+template <int N>
+__global__ void __launch_bounds__(kRowThreads) k_gz_rows(const uint2* __restrict__ gm, int FH,
+                                                         int H, int Hc, int sh, AdjSet set,
+                                                         int rows, const float2* __restrict__ Z,
+                                                         float2* __restrict__ T,
+                                                         const float2* __restrict__ tw) {
+    using C = FFTCfg<N>;
+    constexpr int GPB = kRowThreads / C::TPV;
+    extern __shared__ float lds[];
+    const int grp = group_of<C::TPV>(threadIdx.x), lane = threadIdx.x % C::TPV;
+    const int row = blockIdx.x * GPB + grp;
+    const bool act = row < rows;
+    const int r = act ? row : 0, map = r / Hc, y = r % Hc;
+    const int o = map % kNumOri, entry = map / kNumOri;
+    const CellParams& p = set.cp[entry % set.n];
+    Taps k;
+    k.o = o;
+    k.op = (o + kNumOri / 2) % kNumOri;
+    k.d1 = -2 * p.ea[o] * N + 2 * p.eb[o];
+    k.t = -p.ia[o] * N - p.ib[o];
+    k.rr = p.ra[k.op] * N + p.rb[k.op];
+    const Gather m{gm + (size_t)entry * H * N, FH * N, H * N};
+    const int reach = max(max(abs(k.d1), abs(k.t)), abs(k.rr));
+    const float2* z = Z + (size_t)r * N;
+    float2 v[C::E];
 #pragma unroll
-    for (int o = 0; o < kNumOri; ++o) {
-        const float2 q = Q[(size_t)o * n + i], g = gb[(size_t)o * n + i];
-        re += q.x * g.x + q.y * g.y;
-        im += q.x * g.y - q.y * g.x;
-    }
-    out[t] = make_float2(re * invN, im * invN);
-}
-
-// G_o = invN * G_o * conj(D) in place, per image (G: nb x 8 maps of n, D: nb maps).
-__global__ void k_mul_conjd(float2* __restrict__ G, const float2* __restrict__ D, size_t n,
-                            int nb, float invN) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * nb) return;
-    const size_t b = t / n, i = t - b * n;
-    const float2 d = D[t];
-    float2* gb = G + b * kNumOri * n;
+    for (int e = 0; e < C::E; ++e) v[e] = z[in_index<N>(e, lane)];
+    auto scale = [&](float2& a, float gc) {
+        const float mag = sqrtf(norm1(a));
+        a = scale1(a, mag > 0.f ? gc / mag : 0.f);
+    };
+    // (at most two elements' gathers in flight: all of them would take every register at the
+    // longer lengths; 640 x 480: 1160 us with four, 1085 with two)
+    if (y * N >= reach && (y + 1) * N + reach <= m.HF) {
 #pragma unroll
-    for (int o = 0; o < kNumOri; ++o) {
-        const float2 g = gb[(size_t)o * n + i];
-        gb[(size_t)o * n + i] =
-            make_float2((g.x * d.x + g.y * d.y) * invN, (g.y * d.x - g.x * d.y) * invN);
+        for (int e = 0; e < C::E; ++e) {
+            if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+            scale(v[e], gather_gc<false>(m, k, y * N + in_index<N>(e, lane)));
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) {
+            if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+            scale(v[e], gather_gc<true>(m, k, y * N + in_index<N>(e, lane)));
+        }
+    }
+    bimpdev::fft<N, false>(v, lds + grp * bimpdev::fft_lds_floats<N>(), lane, tw);
+    if (act) {
+        float2* t = T + (size_t)map * Hc * N;
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) t[blk_at(out_index<N>(e, lane), y, Hc, sh)] = v[e];
     }
 }
 
-// Rows (r - kX) mod FH, r = 0..kW-1, of the 8 column-transformed maps Z (FH x FW each) into
-// Yc (8 x kW rows of FW): the only rows of Y_o the parameter partials read.
-__global__ void k_gather_tap_rows(const float2* __restrict__ Z, int kW, int kX, int FH, int FW,
-                                  float2* __restrict__ Yc) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y, o = blockIdx.z;
-    if (x >= FW) return;
-    const int y = (r - kX + FH) % FH;
-    Yc[((size_t)o * kW + r) * FW + x] = Z[((size_t)o * FH + y) * FW + x];
+// Register order of a forward transform's result -> order of an inverse transform's input.
+template <int N>
+__device__ __forceinline__ void to_input_order(float2 (&v)[FFTCfg<N>::E], float2* my, int lane) {
+    using R = bimpdev::RadInfo<typename FFTCfg<N>::Rad>;
+    if constexpr (R::first != R::last) {
+#pragma unroll
+        for (int e = 0; e < FFTCfg<N>::E; ++e) my[out_index<N>(e, lane)] = v[e];
+        bimpdev::stage_sync<FFTCfg<N>::TPV>();
+#pragma unroll
+        for (int e = 0; e < FFTCfg<N>::E; ++e) v[e] = my[in_index<N>(e, lane)];
+        bimpdev::stage_sync<FFTCfg<N>::TPV>();
+    }
+}
+
+// All that happens to the gradient spectra Ghat_o of one column block, which never leave the
+// chip: for each orientation the columns of T (rows [0, Hc), zero below) are transformed;
+// conj(Q_o) Ghat_o adds to the image's spectrum, and Ghat_o conj(D) / (FH*FW) is transformed
+// back for its kW tap rows (r - kX) mod FH, the only ones the parameter sums read, into Yc.
+// Then the image's columns go back, and the rows the clamp padding repeated fold onto rows
+// 0 and H-1 (pad^T in y), so that only H rows remain for the row pass, in block layout in A.
+// Bound by the transforms' VALU work and the read of T; 300 us for four scales of eight
+// 512 x 512 images.  As separate passes over the eight maps the two transforms, the sum and
+// the product took 4 x 142 us.  blockIdx.x: column block.
+template <int N>
+__global__ void __launch_bounds__(ACfg<N>::THREADS) k_adj_cols(const float2* __restrict__ T,
+                                                               const float2* __restrict__ D,
+                                                               AdjSet set, int nb, int W, int H,
+                                                               int Hc, float invN, int kwmax,
+                                                               float2* __restrict__ Yc,
+                                                               float2* __restrict__ Aimg,
+                                                               float2* __restrict__ sums,
+                                                               const float2* __restrict__ tw) {
+    using A = ACfg<N>;
+    extern __shared__ float2 lds2[];
+    // the images of one scale run together and share Q in the L2s
+    const int blk = blockIdx.x, j = blockIdx.y / nb, entry = (int)(blockIdx.y % nb) * set.n + j;
+    const int kW = set.kW[j], kX = set.kX[j];
+    const int g = group_of<A::TPV>(threadIdx.x), lane = threadIdx.x % A::TPV;
+    const int b = threadIdx.x % A::CB, y0 = threadIdx.x / A::CB;
+    const int kx = blk * A::CB + g;
+    const float2* d = D + ((size_t)entry * W + kx) * N;
+    float2* my = lds2 + (size_t)g * A::S;
+    // The running sum over orientations: in registers up to 16 values per lane; above, in
+    // memory (each lane its own elements), since both arrays no longer fit (1536 points: 170
+    // registers spilled).
+    constexpr bool kRegs = A::E <= 16;
+    float2* const sum = sums + ((size_t)entry * W + kx) * N;
+    float2 acc[A::E];
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) acc[e] = make_float2(0.f, 0.f);
+#pragma unroll 1
+    for (int o = 0; o < kNumOri; ++o) {
+        const float2* t = T + (((size_t)entry * kNumOri + o) * W + (size_t)blk * A::CB) * Hc;
+        float2 v[A::E];
+#pragma unroll
+        for (int i = 0; i < A::E; ++i) {
+            const int y = y0 + i * A::TPV;
+            v[i] = y < Hc ? t[(size_t)y * A::CB + b] : make_float2(0.f, 0.f);
+        }
+        __syncthreads();  // the tap rows of the orientation before have left the staging region
+#pragma unroll
+        for (int i = 0; i < A::E; ++i) lds2[b * A::S + y0 + i * A::TPV] = v[i];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < A::E; ++e) v[e] = my[in_index<N>(e, lane)];
+        bimpdev::stage_sync<A::TPV>();
+        bimpdev::fft<N, false>(v, reinterpret_cast<float*>(my), lane, tw);
+        const float2* q = set.Q[j] + ((size_t)o * W + kx) * N;
+#pragma unroll
+        for (int e = 0; e < A::E; ++e) {
+            if (e % 8 == 0) __builtin_amdgcn_sched_barrier(0);  // at most eight loads ahead
+            const int i = out_index<N>(e, lane);
+            const float2 qv = q[i], dv = d[i], gv = v[e];
+            if constexpr (kRegs) {
+                acc[e].x += qv.x * gv.x + qv.y * gv.y;
+                acc[e].y += qv.x * gv.y - qv.y * gv.x;
+            } else {
+                float2 a = o ? sum[i] : make_float2(0.f, 0.f);
+                a.x += qv.x * gv.x + qv.y * gv.y;
+                a.y += qv.x * gv.y - qv.y * gv.x;
+                sum[i] = a;
+            }
+            v[e] = scale1(make_float2(fmaf(gv.x, dv.x, mul1(gv.y, dv.y)),
+                                      fmaf(gv.y, dv.x, -mul1(gv.x, dv.y))), invN);
+        }
+        to_input_order<N>(v, my, lane);
+        bimpdev::fft<N, true>(v, reinterpret_cast<float*>(my), lane, tw);
+#pragma unroll
+        for (int e = 0; e < A::E; ++e) my[out_index<N>(e, lane)] = v[e];
+        __syncthreads();
+        float2* yc = Yc + ((size_t)entry * kNumOri + o) * kwmax * W + (size_t)blk * A::CB + b;
+        for (int r = y0; r < kW; r += A::TPV) {
+            const int y = r < kX ? r - kX + N : r - kX;
+            yc[(size_t)r * W] = lds2[b * A::S + y];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) {
+        if constexpr (!kRegs) acc[e] = sum[out_index<N>(e, lane)];
+        acc[e] = scale1(acc[e], invN);
+    }
+    __syncthreads();
+    to_input_order<N>(acc, my, lane);
+    bimpdev::fft<N, true>(acc, reinterpret_cast<float*>(my), lane, tw);
+    // fold: rows [H, H + kX) onto H - 1, rows [H + kX, N) onto 0, summed over the group's lanes
+    float2 last = make_float2(0.f, 0.f), first = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) {
+        const int y = out_index<N>(e, lane);
+        my[y] = acc[e];
+        if (y >= H && y < H + kX) last = bimpdev::cadd(last, acc[e]);
+        if (y >= H + kX) first = bimpdev::cadd(first, acc[e]);
+    }
+    if (H < N) {
+        constexpr int WL = A::TPV < 64 ? A::TPV : 64;
+#pragma unroll
+        for (int sh = WL / 2; sh >= 1; sh >>= 1) {
+            last.x += __shfl_xor(last.x, sh, WL);
+            last.y += __shfl_xor(last.y, sh, WL);
+            first.x += __shfl_xor(first.x, sh, WL);
+            first.y += __shfl_xor(first.y, sh, WL);
+        }
+        // one lane per wavefront of the group adds its share, one wavefront after the other
+        for (int wv = 0; wv < A::TPV / WL; ++wv) {
+            bimpdev::stage_sync<A::TPV>();
+            if (lane == wv * WL) {
+                my[H - 1] = bimpdev::cadd(my[H - 1], last);
+                my[0] = bimpdev::cadd(my[0], first);
+            }
+        }
+    }
+    __syncthreads();
+    float2* out = Aimg + ((size_t)entry * W + (size_t)blk * A::CB) * H;
+#pragma unroll
+    for (int i = 0; i < A::E; ++i) {
+        const int y = y0 + i * A::TPV;
+        if (y < H) out[(size_t)y * A::CB + b] = lds2[b * A::S + y];
+    }
+}
+
+// Image gradient of one level row: for each scale of the group the inverse row transform of
+// A's row, its real part with the padded columns folded onto columns 0 and W-1 (pad^T in x),
+// scaled and added in the scales' order to the level's gradient (`pitch` floats per row, images
+// lstride apart), which starts at zero with `fresh`; the columns and rows of the level outside
+// the H x W data are then cleared as well.  One group of lanes per (image, row).
+template <int N>
+__global__ void __launch_bounds__(kRowThreads) k_img_rows(const float2* __restrict__ Aimg, int H,
+                                                          int W, int sh, AdjInts k, int nscales,
+                                                          int rows, float s, int fresh,
+                                                          float* __restrict__ gL, int pitch,
+                                                          int lrows, size_t lstride,
+                                                          const float2* __restrict__ tw) {
+    using C = FFTCfg<N>;
+    constexpr int GPB = kRowThreads / C::TPV;
+    constexpr int WL = C::TPV < 64 ? C::TPV : 64;
+    extern __shared__ float lds[];
+    __shared__ float2 part[GPB][2];
+    const int grp = group_of<C::TPV>(threadIdx.x), lane = threadIdx.x % C::TPV;
+    const int row = blockIdx.x * GPB + grp;
+    const bool act = row < rows;
+    const int r = act ? row : 0, img = r / H, y = r % H;
+    float* g = gL + img * lstride + (size_t)y * pitch;
+    float sum[C::E];
+#pragma unroll
+    for (int e = 0; e < C::E; ++e) {
+        const int x = out_index<N>(e, lane);
+        sum[e] = !fresh && x < W ? g[x] : 0.f;
+    }
+#pragma unroll 1
+    for (int j = 0; j < nscales; ++j) {
+        const float2* a = Aimg + (size_t)(img * nscales + j) * H * N;
+        const int kX = k.v[j];
+        float2 v[C::E];
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) v[e] = a[blk_at(in_index<N>(e, lane), y, H, sh)];
+        bimpdev::fft<N, true>(v, lds + grp * bimpdev::fft_lds_floats<N>(), lane, tw);
+        float last = 0.f, first = 0.f;
+        if (W < N) {
+#pragma unroll
+            for (int e = 0; e < C::E; ++e) {
+                const int x = out_index<N>(e, lane);
+                if (x >= W && x < W + kX) last += v[e].x;
+                if (x >= W + kX) first += v[e].x;
+            }
+#pragma unroll
+            for (int d = WL / 2; d >= 1; d >>= 1) {
+                last += __shfl_xor(last, d, WL);
+                first += __shfl_xor(first, d, WL);
+            }
+            if constexpr (C::TPV > 64) {
+                __syncthreads();
+                if (lane % 64 == 0) part[grp][lane / 64] = make_float2(last, first);
+                __syncthreads();
+                last = part[grp][0].x + part[grp][1].x;
+                first = part[grp][0].y + part[grp][1].y;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) {
+            const int x = out_index<N>(e, lane);
+            float t = v[e].x;
+            if (x == W - 1) t += last;
+            if (x == 0) t += first;
+            sum[e] += s * t;
+        }
+    }
+    if (!act) return;
+#pragma unroll
+    for (int e = 0; e < C::E; ++e) {
+        const int x = out_index<N>(e, lane);
+        if (x < W) g[x] = sum[e];
+    }
+    if (fresh) {
+        for (int x = W + lane; x < pitch; x += C::TPV) g[x] = 0.f;
+        if (y == H - 1)
+            for (int i = lane; i < (lrows - H) * pitch; i += C::TPV) g[pitch + i] = 0.f;
+    }
+}
+
+// Row transforms of the tap rows: rows r < kW of the 8 x kwmax rows of each entry, in place.
+template <int N>
+__global__ void __launch_bounds__(kRowThreads) k_tap_rows(float2* __restrict__ Yc, AdjInts kW,
+                                                          int nscales, int kwmax, int rows,
+                                                          const float2* __restrict__ tw) {
+    using C = FFTCfg<N>;
+    constexpr int GPB = kRowThreads / C::TPV;
+    extern __shared__ float lds[];
+    const int grp = group_of<C::TPV>(threadIdx.x), lane = threadIdx.x % C::TPV;
+    const int row = blockIdx.x * GPB + grp;
+    const int r = row < rows ? row : 0;
+    const int entry = r / (kNumOri * kwmax);
+    // (a 128-lane group's stages take the workgroup barrier: unused rows are transformed too)
+    const bool act = row < rows && r % kwmax < kW.v[entry % nscales];
+    float2* p = Yc + (size_t)r * N;
+    float2 v[C::E];
+#pragma unroll
+    for (int e = 0; e < C::E; ++e)
+        v[e] = act ? p[in_index<N>(e, lane)] : make_float2(0.f, 0.f);
+    bimpdev::fft<N, true>(v, lds + grp * bimpdev::fft_lds_floats<N>(), lane, tw);
+    if (act) {
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) p[out_index<N>(e, lane)] = v[e];
+    }
 }
 
 // Parameter gradient partials: sum over orientations and taps of
 //   Re Y_o(tap) dKe/dtheta + Im Y_o(tap) dKo/dtheta  for theta = (sigma ratio, gamma),
-// with Y_o's tap rows in Yc (k_gather_tap_rows, then row transforms); one pair of partial
-// sums per block (fixed-order tree), summed on the host in block order.
-__global__ void __launch_bounds__(256) k_param_partials(const float2* __restrict__ Yc, int kW,
-                                                        int kX, int FW,
-                                                        const float* __restrict__ dK,
+// with Y_o's tap rows in Yc; one pair of partial sums per block (fixed-order tree), summed on
+// the host in block order.  blockIdx.y: entry; scale j's partials start at j * jstride.
+__global__ void __launch_bounds__(256) k_param_partials(const float2* __restrict__ Yc, AdjSet set,
+                                                        int kwmax, int FW,
                                                         float* __restrict__ partials,
-                                                        size_t pstride) {
+                                                        size_t pstride, int jstride) {
     __shared__ float sr[256], sg[256];
+    const int entry = blockIdx.y, j = entry % set.n;
+    const int kW = set.kW[j], kX = set.kX[j];
+    const float* dK = set.dK[j];
     const int n = kNumOri * kW * kW;
+    if ((int)blockIdx.x * 256 >= n) return;
     const int i = blockIdx.x * 256 + threadIdx.x;
-    // blockIdx.y: image of the batch (its tap rows and its partials)
-    Yc += (size_t)blockIdx.y * kNumOri * kW * FW;
-    partials += (size_t)blockIdx.y * pstride;
+    Yc += (size_t)entry * kNumOri * kwmax * FW;
+    partials += (size_t)(entry / set.n) * pstride + (size_t)j * jstride;
     float vr = 0.f, vg = 0.f;
     if (i < n) {
         const int o = i / (kW * kW), m = i % (kW * kW), r = m / kW, c = m % kW;
         const int x = (c - kX + FW) % FW;
-        const float2 v = Yc[((size_t)o * kW + r) * FW + x];
+        const float2 v = Yc[((size_t)o * kwmax + r) * FW + x];
         const size_t stride = (size_t)n;
         vr = v.x * dK[0 * stride + i] + v.y * dK[1 * stride + i];
         vg = v.x * dK[2 * stride + i] + v.y * dK[3 * stride + i];
@@ -471,22 +782,40 @@ inline dim3 ew(size_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
 }  // namespace
 
+// Dynamic LDS of the row kernels (kRowThreads / TPV exchange regions) and column kernels.
+template <int N>
+constexpr int row_lds() {
+    return (kRowThreads / FFTCfg<N>::TPV) * bimpdev::fft_lds_floats<N>() * (int)sizeof(float);
+}
+template <int N>
+int row_blocks(int rows) {
+    constexpr int GPB = kRowThreads / FFTCfg<N>::TPV;
+    return (rows + GPB - 1) / GPB;
+}
+int block_shift(int n) {
+    int sh = 0;
+    while ((1 << sh) < diff_block_columns(n)) ++sh;
+    return sh;
+}
+
 hipError_t diff_prepare(int n) {
 #define X(N)                                                                                 \
     if (n == N) {                                                                            \
-        const int lds = (kRowThreads / FFTCfg<N>::TPV) * bimpdev::fft_lds_floats<N>() * (int)sizeof(float); \
-        const int clds = CColCfg<N>::CB * CColCfg<N>::S * (int)sizeof(float2);               \
-        hipError_t e = hipFuncSetAttribute((const void*)k_c2c_rows<N, false>,                \
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
-        if (e == hipSuccess)                                                                 \
-            e = hipFuncSetAttribute((const void*)k_c2c_rows<N, true>,                        \
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds);        \
-        if (e == hipSuccess)                                                                 \
-            e = hipFuncSetAttribute((const void*)k_c2c_cols<N, false>,                       \
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, clds);       \
-        if (e == hipSuccess)                                                                 \
-            e = hipFuncSetAttribute((const void*)k_c2c_cols<N, true>,                        \
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, clds);       \
+        const std::pair<const void*, int> f[] = {                                            \
+            {(const void*)k_c2c_rows<N, false>, row_lds<N>()},                               \
+            {(const void*)k_pad_rows<N>, row_lds<N>()},                                      \
+            {(const void*)k_z_rows<N>, row_lds<N>()},                                        \
+            {(const void*)k_gz_rows<N>, row_lds<N>()},                                       \
+            {(const void*)k_img_rows<N>, row_lds<N>()},                                      \
+            {(const void*)k_tap_rows<N>, row_lds<N>()},                                      \
+            {(const void*)k_cols_kx<N>, ACfg<N>::LDS},                                       \
+            {(const void*)k_z_cols<N>, ACfg<N>::LDS},                                        \
+            {(const void*)k_adj_cols<N>, ACfg<N>::LDS}};                                     \
+        hipError_t e = hipSuccess;                                                           \
+        for (const auto& k : f)                                                              \
+            if (e == hipSuccess)                                                             \
+                e = hipFuncSetAttribute(k.first, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                        k.second);                                           \
         return e;                                                                            \
     }
     BIMP_FOR_SIZES(X)
@@ -494,21 +823,11 @@ hipError_t diff_prepare(int n) {
     return hipErrorInvalidValue;
 }
 
-hipError_t diff_rows_maps(float2* data, int maps, int per_map, size_t map_stride, int n,
-                          bool inv, const float2* tw, hipStream_t s) {
-    const int rows = maps * per_map;
-    if (maps < 1 || per_map < 1) return hipErrorInvalidValue;
+hipError_t diff_rows(float2* data, int rows, int n, const float2* tw, hipStream_t s) {
 #define X(N)                                                                                 \
     if (n == N) {                                                                            \
-        constexpr int GPB = kRowThreads / FFTCfg<N>::TPV;                                    \
-        const int lds = GPB * bimpdev::fft_lds_floats<N>() * (int)sizeof(float);             \
-        dim3 grid((rows + GPB - 1) / GPB);                                                   \
-        if (inv)                                                                             \
-            k_c2c_rows<N, true><<<grid, kRowThreads, lds, s>>>(data, rows, per_map, map_stride, \
-                                                               tw);                          \
-        else                                                                                 \
-            k_c2c_rows<N, false><<<grid, kRowThreads, lds, s>>>(data, rows, per_map,         \
-                                                                map_stride, tw);             \
+        k_c2c_rows<N, false><<<row_blocks<N>(rows), kRowThreads, row_lds<N>(), s>>>(data, rows, \
+                                                                                    tw);     \
         return hipGetLastError();                                                            \
     }
     BIMP_FOR_SIZES(X)
@@ -516,21 +835,14 @@ hipError_t diff_rows_maps(float2* data, int maps, int per_map, size_t map_stride
     return hipErrorInvalidValue;
 }
 
-hipError_t diff_rows(float2* data, int rows, int n, bool inv, const float2* tw, hipStream_t s) {
-    return diff_rows_maps(data, 1, rows, 0, n, inv, tw, s);
-}
-
-hipError_t diff_cols(float2* data, int n, int w, int batch, bool inv, const float2* tw,
-                     hipStream_t s) {
+hipError_t diff_cols_kx(const float2* in, int H, int FH, int W, const AdjInts& k, int nscales,
+                        int maps, float2* out, const float2* tw, hipStream_t s) {
 #define X(N)                                                                                 \
-    if (n == N) {                                                                            \
-        using CC = CColCfg<N>;                                                               \
-        const int lds = CC::CB * CC::S * (int)sizeof(float2);                                \
-        dim3 grid((w + CC::CB - 1) / CC::CB, batch);                                         \
-        if (inv)                                                                             \
-            k_c2c_cols<N, true><<<grid, CC::THREADS, lds, s>>>(data, w, tw);                 \
-        else                                                                                 \
-            k_c2c_cols<N, false><<<grid, CC::THREADS, lds, s>>>(data, w, tw);                \
+    if (FH == N) {                                                                           \
+        using A = ACfg<N>;                                                                   \
+        if (W % A::CB) return hipErrorInvalidValue;                                          \
+        k_cols_kx<N><<<dim3(W / A::CB, maps), A::THREADS, A::LDS, s>>>(in, H, W, k, nscales, \
+                                                                        out, tw);            \
         return hipGetLastError();                                                            \
     }
     BIMP_FOR_SIZES(X)
@@ -550,22 +862,9 @@ hipError_t diff_pyr_down_adj(const float* gdst, int dw, int dh, float* gsrc, int
     return hipGetLastError();
 }
 
-hipError_t diff_pad(const float* L, int pitch, size_t lstride, int H, int W, int FH, int FW,
-                    int k, float sc, float2* out, int nb, hipStream_t s) {
-    k_pad_fwd<<<dim3((FW + 127) / 128, FH, nb), 128, 0, s>>>(L, pitch, lstride, H, W, FH, FW, k,
-                                                             sc, out);
-    return hipGetLastError();
-}
-
-hipError_t diff_pad_adj(const float2* g, int H, int W, int FH, int FW, int k, float sc,
-                        float* gL, int pitch, size_t lstride, int nb, hipStream_t s) {
-    k_pad_adj<<<dim3((W + 127) / 128, H, nb), 128, 0, s>>>(g, H, W, FH, FW, k, sc, gL, pitch,
-                                                           lstride);
-    return hipGetLastError();
-}
-
 hipError_t diff_q_to_g(const float2* Q, int FH, int FW, float invN, float* G, hipStream_t s) {
-    k_q_to_g<<<dim3((FW + 31) / 32, (FH + 31) / 32, kUniqueOri), 256, 0, s>>>(Q, FH, FW, invN, G);
+    const size_t n = (size_t)kUniqueOri * FH * FW;
+    k_q_to_g<<<ew(n), 256, 0, s>>>(Q, n, invN, G);
     return hipGetLastError();
 }
 
@@ -575,61 +874,91 @@ hipError_t diff_bank_pad(const float* ke, const float* ko, int kW, int kX, int F
     return hipGetLastError();
 }
 
-hipError_t diff_spec_mul(const float2* D, const float2* Q, float2* Z, size_t n, int nb,
-                         float invN, hipStream_t s) {
-    k_spec_mul<<<ew(n * nb), 256, 0, s>>>(D, Q, Z, n, nb, invN);
-    return hipGetLastError();
+hipError_t diff_backward_rows(const AdjSet& set, const AdjLevel& L, const AdjBuffers& B,
+                              const float2* tw, hipStream_t s) {
+    const int entries = set.n * L.nb;
+    const int prows = entries * L.H;
+#define X(N)                                                                                 \
+    if (L.FW == N) {                                                                         \
+        k_pad_rows<N><<<row_blocks<N>(prows), kRowThreads, row_lds<N>(), s>>>(               \
+            L.img, L.pitch, L.lstride, L.H, L.W, set.ints(set.kX), set.n, L.gain, prows, B.T, tw); \
+        return hipGetLastError();                                                            \
+    }
+    BIMP_FOR_SIZES(X)
+#undef X
+    return hipErrorInvalidValue;
 }
 
-hipError_t diff_mag(const float2* Z, float* C, size_t n, hipStream_t s) {
-    k_mag<<<ew(n), 256, 0, s>>>(Z, C, n);
-    return hipGetLastError();
+hipError_t diff_z_cols(const AdjSet& set, const AdjLevel& L, const AdjBuffers& B, const float2* tw,
+                       hipStream_t s) {
+#define X(N)                                                                                 \
+    if (L.FH == N) {                                                                         \
+        using A = ACfg<N>;                                                                   \
+        const int per = (L.FW / A::CB + 7) / 8;                                              \
+        k_z_cols<N><<<8 * kNumOri * per * set.n * L.nb, A::THREADS, A::LDS, s>>>(            \
+            B.D, set, L.nb, L.FW, L.Hc, L.invN, B.T, tw);                                    \
+        return hipGetLastError();                                                            \
+    }
+    BIMP_FOR_SIZES(X)
+#undef X
+    return hipErrorInvalidValue;
 }
 
-hipError_t diff_cells_adj(const float* C, int FH, int FW, int H, int W, const CellParams& p,
-                          const float* gD, size_t gstride, float* Wm, float* gC, int nb,
-                          hipStream_t s) {
-    k_cells_adj_w<<<dim3((FW + 127) / 128, FH, nb), 128, 0, s>>>(C, FH, FW, H, W, p, gD, gstride,
-                                                                 Wm);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    k_cells_adj_g<<<dim3((FW + 127) / 128, FH, kNumOri * nb), 128, 0, s>>>(Wm, FH, FW, p, gC);
-    return hipGetLastError();
+hipError_t diff_cells_grad(const AdjSet& set, const AdjLevel& L, const AdjBuffers& B,
+                           const float* gD, size_t gstride, const float2* tw, hipStream_t s) {
+    const int entries = set.n * L.nb, rows = entries * kNumOri * L.Hc;
+    const int sh = block_shift(L.FH);
+#define X(N)                                                                                 \
+    if (L.FW == N) {                                                                         \
+        k_z_rows<N><<<row_blocks<N>(rows), kRowThreads, row_lds<N>(), s>>>(B.T, L.Hc, sh, rows, \
+                                                                           B.Z, B.C, tw);    \
+        k_branch_bits<<<dim3((N + 255) / 256, L.H, entries), 256, 0, s>>>(                   \
+            B.C, L.Hc, L.FH, N, L.H, L.W, set, gD, gstride, B.gm);                           \
+        k_gz_rows<N><<<row_blocks<N>(rows), kRowThreads, row_lds<N>(), s>>>(                 \
+            B.gm, L.FH, L.H, L.Hc, sh, set, rows, B.Z, B.T, tw);                             \
+        return hipGetLastError();                                                            \
+    }
+    BIMP_FOR_SIZES(X)
+#undef X
+    return hipErrorInvalidValue;
 }
 
-hipError_t diff_grad_z(const float* gC, float2* Z, size_t n, hipStream_t s) {
-    k_grad_z<<<ew(n), 256, 0, s>>>(gC, Z, n);
-    return hipGetLastError();
+hipError_t diff_adj_cols(const AdjSet& set, const AdjLevel& L, const AdjBuffers& B, int kwmax,
+                         const float2* tw, hipStream_t s) {
+#define X(N)                                                                                 \
+    if (L.FH == N) {                                                                         \
+        using A = ACfg<N>;                                                                   \
+        k_adj_cols<N><<<dim3(L.FW / A::CB, set.n * L.nb), A::THREADS, A::LDS, s>>>(          \
+            B.T, B.D, set, L.nb, L.FW, L.H, L.Hc, L.invN, kwmax, B.Yc, B.A, B.Z, tw);        \
+        return hipGetLastError();                                                            \
+    }
+    BIMP_FOR_SIZES(X)
+#undef X
+    return hipErrorInvalidValue;
 }
 
-hipError_t diff_accum_conjq(const float2* Q, const float2* G, float2* out, size_t n, int nb,
-                            float invN, hipStream_t s) {
-    k_accum_conjq<<<ew(n * nb), 256, 0, s>>>(Q, G, out, n, nb, invN);
-    return hipGetLastError();
-}
-
-hipError_t diff_mul_conjd(float2* G, const float2* D, size_t n, int nb, float invN,
-                          hipStream_t s) {
-    k_mul_conjd<<<ew(n * nb), 256, 0, s>>>(G, D, n, nb, invN);
-    return hipGetLastError();
+hipError_t diff_adj_rows(const AdjSet& set, const AdjLevel& L, const AdjBuffers& B, int kwmax,
+                         bool fresh, float* glev, int lrows, float* partials, size_t pstride,
+                         int jstride, const float2* tw, hipStream_t s) {
+    const int entries = set.n * L.nb, rows = L.nb * L.H, trows = entries * kNumOri * kwmax;
+    const int sh = block_shift(L.FH);
+#define X(N)                                                                                 \
+    if (L.FW == N) {                                                                         \
+        k_img_rows<N><<<row_blocks<N>(rows), kRowThreads, row_lds<N>(), s>>>(                \
+            B.A, L.H, L.W, sh, set.ints(set.kX), set.n, rows, L.gain, fresh ? 1 : 0, glev,   \
+            L.pitch, lrows, L.lstride, tw);                                                  \
+        k_tap_rows<N><<<row_blocks<N>(trows), kRowThreads, row_lds<N>(), s>>>(               \
+            B.Yc, set.ints(set.kW), set.n, kwmax, trows, tw);                                \
+        k_param_partials<<<dim3(diff_param_blocks(kwmax), entries), 256, 0, s>>>(            \
+            B.Yc, set, kwmax, N, partials, pstride, jstride);                                \
+        return hipGetLastError();                                                            \
+    }
+    BIMP_FOR_SIZES(X)
+#undef X
+    return hipErrorInvalidValue;
 }
 
 int diff_param_blocks(int kW) { return (kNumOri * kW * kW + 255) / 256; }
-
-hipError_t diff_gather_tap_rows(const float2* Z, int kW, int kX, int FH, int FW, float2* Yc,
-                                int nb, hipStream_t s) {
-    // map index z = image * 8 + orientation in both Z and Yc
-    k_gather_tap_rows<<<dim3((FW + 127) / 128, kW, kNumOri * nb), 128, 0, s>>>(Z, kW, kX, FH, FW,
-                                                                               Yc);
-    return hipGetLastError();
-}
-
-hipError_t diff_param_partials(const float2* Yc, int kW, int kX, int FW, const float* dK,
-                               float* partials, size_t pstride, int nb, hipStream_t s) {
-    k_param_partials<<<dim3(diff_param_blocks(kW), nb), 256, 0, s>>>(Yc, kW, kX, FW, dK, partials,
-                                                                     pstride);
-    return hipGetLastError();
-}
 
 hipError_t diff_fill(float* p, size_t n, hipStream_t s) {
     k_fill<<<ew(n), 256, 0, s>>>(p, n);
