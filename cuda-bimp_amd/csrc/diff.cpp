@@ -57,7 +57,8 @@ struct bimp_diff {
     float2 *R = nullptr, *T = nullptr;  // forward: row spectra and inverse-column output
     float* Sf = nullptr;                // forward: single-stopped maps (scratch)
     size_t rSize = 0, tSize = 0;
-    float* taps = nullptr;              // Ke, Ko of the scale being set up
+    float2* taps = nullptr;             // (Ke, Ko) of a group being set up, per scale
+    size_t tapStride = 0;
     unsigned* maxslot = nullptr;
     // backward: work buffers of up to `entries` (scale, image) pairs per launch
     bimpk::AdjBuffers adj{};
@@ -82,35 +83,39 @@ int dfail(bimp_diff* d, int code, const std::string& m) {
             return dfail(d, BIMP_E_DEVICE, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+// Taps, tap derivatives and bank spectra of (ratio, gamma), on the device.
 int set_params(bimp_diff* d, float ratio, float gamma, hipStream_t s) {
-    for (auto& x : d->sc) {
-        const auto& g = x.g;
-        const int kk = g.kW * g.kW;
-        std::vector<float> ke((size_t)kNumOri * kk), ko((size_t)kNumOri * kk);
-        std::vector<float> dk((size_t)4 * kNumOri * kk);
-        std::vector<double> a(kk), b(kk), c(kk), e(kk);
-        for (int o = 0; o < kNumOri; ++o) {
-            bimph::gabor_taps(g, o, gamma, ratio, ke.data() + (size_t)o * kk, ko.data() + (size_t)o * kk);
-            bimph::gabor_taps_grad(g, o, gamma, ratio, a.data(), b.data(), c.data(), e.data());
-            const size_t n = (size_t)kNumOri * kk;
-            for (int m = 0; m < kk; ++m) {
-                dk[0 * n + (size_t)o * kk + m] = (float)a[m];
-                dk[1 * n + (size_t)o * kk + m] = (float)b[m];
-                dk[2 * n + (size_t)o * kk + m] = (float)c[m];
-                dk[3 * n + (size_t)o * kk + m] = (float)e[m];
-            }
-        }
-        DCHK(d, hipMemcpy(d->taps, ke.data(), ke.size() * 4, hipMemcpyHostToDevice));
-        DCHK(d, hipMemcpy(d->taps + ke.size(), ko.data(), ko.size() * 4, hipMemcpyHostToDevice));
-        DCHK(d, hipMemcpy(x.dK, dk.data(), dk.size() * 4, hipMemcpyHostToDevice));
-        float2* const rows = d->adj.T;  // free here: no pass of this context is under way
-        DCHK(d, bimpk::diff_bank_pad(d->taps, d->taps + ke.size(), g.kW, g.kX, g.FH, g.FW, rows, s));
-        DCHK(d, bimpk::diff_rows(rows, kNumOri * g.FH, g.FW, d->tw[g.FW], s));
-        DCHK(d, bimpk::diff_cols_kx(rows, g.FH, g.FH, g.FW, bimpk::AdjInts{}, 1, kNumOri, x.Q,
-                                    d->tw[g.FH], s));
-        DCHK(d, bimpk::diff_q_to_g(x.Q, g.FH, g.FW, 1.0f / ((float)g.FH * (float)g.FW), x.G, s));
-        DCHK(d, hipStreamSynchronize(s));
+    const double pi = 3.1415926535897932384626433832795;
+    bimpk::TapTrig trig;
+    for (int o = 0; o < kNumOri; ++o) {
+        const float theta = (float)(o * pi / 8);
+        trig.st[o] = (float)std::sin((double)theta);
+        trig.ct[o] = (float)std::cos((double)theta);
+        trig.std[o] = std::sin(o * pi / 8);
+        trig.ctd[o] = std::cos(o * pi / 8);
     }
+    for (const auto& gr : d->groups) {
+        // (the tap rows of `entries` scales fit the work buffer they pass through)
+        for (int j0 = 0; j0 < gr.second; j0 += d->entries) {
+            bimpk::TapSet set{};
+            set.n = std::min(gr.second - j0, d->entries);
+            for (int j = 0; j < set.n; ++j) {
+                const DScale& x = d->sc[gr.first + j0 + j];
+                const double sigma = (double)x.g.lambda * (double)ratio;
+                const float sf = (float)sigma, sq = sf * sf;
+                set.s[j] = bimpk::TapScale{x.g.lambda, x.g.fs, -1.0f / (2 * sq), sigma, x.g.kW,
+                                           x.g.kX, x.dK, x.Q, x.G};
+            }
+            const auto& g = d->sc[gr.first].g;
+            DCHK(d, bimpk::diff_taps(set, trig, gamma, d->taps, d->tapStride, s));
+            // T is free here: no pass of this context is under way
+            DCHK(d, bimpk::diff_bank_rows(set, d->taps, d->tapStride, d->kwMax, g.FW, d->adj.T,
+                                          d->tw[g.FW], s));
+            DCHK(d, bimpk::diff_bank_cols(set, d->adj.T, d->kwMax, g.FH, g.FW,
+                                          1.0f / ((float)g.FH * (float)g.FW), d->tw[g.FH], s));
+        }
+    }
+    DCHK(d, hipStreamSynchronize(s));
     d->ratio = ratio;
     d->gamma = gamma;
     return BIMP_OK;
@@ -316,10 +321,9 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
         if (hipMalloc(&d->lev[l], NB * d->lw[l] * d->lh[l] * 4) != hipSuccess ||
             hipMalloc(&d->glev[l], NB * d->lw[l] * d->lh[l] * 4) != hipSuccess)
             return bail(BIMP_E_ALLOC);
-    size_t maxTaps = 0;
     for (auto& x : d->sc) {
         const size_t kk = (size_t)x.g.kW * x.g.kW;
-        maxTaps = std::max(maxTaps, kk);
+        d->tapStride = std::max(d->tapStride, kNumOri * kk);
         d->maxBlocks = std::max(d->maxBlocks, bimpk::diff_param_blocks(x.g.kW));
         if (hipMalloc(&x.Q, (size_t)kNumOri * x.g.FH * x.g.FW * sizeof(float2)) != hipSuccess ||
             hipMalloc(&x.G, (size_t)bimpk::kUniqueOri * x.g.FH * x.g.FW * sizeof(float)) != hipSuccess ||
@@ -336,7 +340,7 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
         hipMalloc(&w.C, NE * kNumOri * pm * sizeof(float)) != hipSuccess ||
         hipMalloc(&w.gm, NE * pm * sizeof(uint2)) != hipSuccess ||
         hipMalloc(&w.Yc, NE * kNumOri * d->kwMax * kwfw * sizeof(float2)) != hipSuccess ||
-        hipMalloc(&d->taps, 2 * kNumOri * maxTaps * sizeof(float)) != hipSuccess ||
+        hipMalloc(&d->taps, (size_t)bimpk::kAdjMax * d->tapStride * sizeof(float2)) != hipSuccess ||
         hipMalloc(&d->maxslot, sizeof(unsigned)) != hipSuccess ||
         hipMalloc(&d->R, d->rSize * sizeof(float2)) != hipSuccess ||
         hipMalloc(&d->T, d->tSize * sizeof(float2)) != hipSuccess ||

@@ -40,27 +40,12 @@ __device__ __forceinline__ int group_of(int tid) {
     return TPV >= 64 ? __builtin_amdgcn_readfirstlane(tid / TPV) : tid / TPV;
 }
 
-// In-place complex transforms of `rows` contiguous rows of length N.
-template <int N, bool INV>
-__global__ void __launch_bounds__(kRowThreads) k_c2c_rows(float2* __restrict__ data, int rows,
-                                                          const float2* __restrict__ tw) {
-    using C = FFTCfg<N>;
-    constexpr int GPB = kRowThreads / C::TPV;
-    extern __shared__ float lds[];
-    const int grp = group_of<C::TPV>(threadIdx.x), lane = threadIdx.x % C::TPV;
-    // every group transforms (a spare one row 0, unstored): a 128-lane group's stages take
-    // the workgroup barrier
-    const int row = blockIdx.x * GPB + grp;
-    const bool act = row < rows;
-    float2* p = data + (size_t)(act ? row : 0) * N;
-    float2 v[C::E];
+// A transform's results made opaque: what is done with them next would otherwise change how the
+// compiler contracts the transform's last additions, and with that the bits of a spectrum.
+template <int E>
+__device__ __forceinline__ void pin(float2 (&v)[E]) {
 #pragma unroll
-    for (int e = 0; e < C::E; ++e) v[e] = p[in_index<N>(e, lane)];
-    bimpdev::fft<N, INV>(v, lds + grp * bimpdev::fft_lds_floats<N>(), lane, tw);
-    if (act) {
-#pragma unroll
-        for (int e = 0; e < C::E; ++e) p[out_index<N>(e, lane)] = v[e];
-    }
+    for (int e = 0; e < E; ++e) asm volatile("" : "+v"(v[e].x), "+v"(v[e].y));
 }
 
 // Column kernels: a workgroup owns CB adjacent columns, one group of TPV lanes each; a column
@@ -178,27 +163,166 @@ __global__ void k_pyr_down_adj(const float* __restrict__ gdst, int dw, int dh,
     gsrc[(size_t)y * sw + x] += acc;
 }
 
-// G_o(ky, kx) = Re Q_o(ky, kx) / (FH*FW) for o = 0..4, kx-major like Q: the quadrature bank of
-// the detection path's inverse column pass, from the spectra Q of the current parameters.
-__global__ void k_q_to_g(const float2* __restrict__ Q, size_t n, float invN,
-                         float* __restrict__ G) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) G[i] = Q[i].x * invN;
+// ---------------------------------------------------------------- bank of the parameters
+// Taps of the quadrature kernels and their derivatives for one (scale, orientation) per
+// workgroup, by the formulas of the detection path's FP32 taps (cuda_bimp.cu:304-331: FP32
+// expressions around FP64 exp and cos, a sequential FP32 sum of the even taps) and their FP64
+// derivatives, operation for operation as the host evaluates them, with no contraction.  The
+// three sums run in tap order, each on a wavefront of its own over the chunk in LDS.  Bound by
+// FP64 exp and cos; on one host thread the taps of eight scales took 4 ms per parameter change.
+struct TapVals {
+    float e, ko;             // even tap before its DC offset, odd tap
+    double der, deg, dor, dog;  // derivatives by sigma ratio and gamma (even: before their DC)
+};
+__device__ TapVals tap_at(const TapScale& t, const TapTrig& g, int o, float gamma, int row,
+                          int col) {
+#pragma clang fp contract(off)
+    const float phi = (float)(-3.1415926535897932384626433832795 / 2);
+    const int x = col - t.kX, y = row - t.kX;
+    const float xr = (float)x * g.ct[o] + (float)y * g.st[o];
+    const float yr = (float)y * g.ct[o] - (float)x * g.st[o];
+    const float q = xr * xr + gamma * yr * yr;
+    const float env = (float)exp((double)(t.negInv * q));
+    const double f = 2 * 3.1415926535897932384626433832795 * (double)xr / (double)t.lambda;
+    TapVals v;
+    v.e = (float)((double)env * cos(f));
+    v.ko = (float)((double)env * cos(f + (double)phi));
+    const double xd = x, yd = y;
+    const double xrd = xd * g.ctd[o] + yd * g.std[o], yrd = yd * g.ctd[o] - xd * g.std[o];
+    const double qd = xrd * xrd + (double)gamma * yrd * yrd;
+    const double sg = t.sigma;
+    const double envd = exp(-qd / (2 * sg * sg));
+    const double fd = 2 * 3.1415926535897932384626433832795 * xrd / (double)t.lambda;
+    const double phid = -3.1415926535897932384626433832795 / 2;
+    const double dr = envd * qd * (double)t.lambda / (sg * sg * sg);
+    const double dg = -envd * yrd * yrd / (2 * sg * sg);
+    const double ce = cos(fd), co = cos(fd + phid);
+    v.der = dr * ce;
+    v.deg = dg * ce;
+    v.dor = dr * co;
+    v.dog = dg * co;
+    return v;
 }
 
-// Padded complex kernels of the 8 orientations: tap (r, c) sits at ((r-kX) mod FH,
-// (c-kX) mod FW) (requires kW <= FH, FW, so positions are distinct).
-__global__ void k_bank_pad(const float* __restrict__ ke, const float* __restrict__ ko, int kW,
-                           int kX, int FH, int FW, float2* __restrict__ out) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, o = blockIdx.z;
-    if (x >= FW) return;
-    const int r = (y + kX) % FH, c = (x + kX) % FW;
-    float2 v = make_float2(0.f, 0.f);
-    if (r < kW && c < kW) {
-        const size_t m = ((size_t)o * kW + r) * kW + c;
-        v = make_float2(ke[m], ko[m]);
+constexpr int kTapThreads = 1024;
+__global__ void __launch_bounds__(kTapThreads) k_taps(TapSet set, TapTrig trig, float gamma,
+                                                      float2* __restrict__ taps, size_t stride) {
+#pragma clang fp contract(off)
+    __shared__ float ce[kTapThreads];
+    __shared__ double cr[kTapThreads], cg[kTapThreads];
+    __shared__ double sums[3];
+    const int o = blockIdx.x, j = blockIdx.y, tid = threadIdx.x;
+    const TapScale& t = set.s[j];
+    const int kk = t.kW * t.kW;
+    const size_t n = (size_t)kNumOri * kk;
+    float2* out = taps + (size_t)j * stride + (size_t)o * kk;
+    float* dK = t.dK + (size_t)o * kk;
+    float es = 0.f;
+    double ds = 0.0;
+    for (int m0 = 0; m0 < kk; m0 += kTapThreads) {
+        const int m = m0 + tid;
+        if (m < kk) {
+            const TapVals v = tap_at(t, trig, o, gamma, m / t.kW, m % t.kW);
+            out[m] = make_float2(v.e, v.ko);
+            dK[1 * n + m] = (float)v.dor;
+            dK[3 * n + m] = (float)v.dog;
+            ce[tid] = v.e;
+            cr[tid] = v.der;
+            cg[tid] = v.deg;
+        }
+        __syncthreads();
+        const int c = min(kTapThreads, kk - m0);
+        if (tid == 0)
+            for (int i = 0; i < c; ++i) es += ce[i];
+        else if (tid == 64)
+            for (int i = 0; i < c; ++i) ds += cr[i];
+        else if (tid == 128)
+            for (int i = 0; i < c; ++i) ds += cg[i];
+        __syncthreads();
     }
-    out[((size_t)o * FH + y) * FW + x] = v;
+    if (tid == 0) sums[0] = (double)(es / (t.fs * t.fs));
+    if (tid == 64) sums[1] = ds / ((double)t.fs * (double)t.fs);
+    if (tid == 128) sums[2] = ds / ((double)t.fs * (double)t.fs);
+    __syncthreads();
+    const float dc = (float)sums[0];
+    for (int m = tid; m < kk; m += kTapThreads) {
+        const TapVals v = tap_at(t, trig, o, gamma, m / t.kW, m % t.kW);
+        out[m].x = v.e - dc;
+        dK[0 * n + m] = (float)(v.der - sums[1]);
+        dK[2 * n + m] = (float)(v.deg - sums[2]);
+    }
+}
+
+// Row transforms of the kernels placed on the torus, tap (r, c) at ((r-kX) mod FH,
+// (c-kX) mod FW): the kW rows that hold taps (requires kW <= FH, FW).
+template <int N>
+__global__ void __launch_bounds__(kRowThreads) k_bank_rows(const float2* __restrict__ taps,
+                                                           size_t stride, TapSet set, int kwmax,
+                                                           int rows, float2* __restrict__ out,
+                                                           const float2* __restrict__ tw) {
+    using C = FFTCfg<N>;
+    constexpr int GPB = kRowThreads / C::TPV;
+    extern __shared__ float lds[];
+    const int grp = group_of<C::TPV>(threadIdx.x), lane = threadIdx.x % C::TPV;
+    const int row = blockIdx.x * GPB + grp;
+    const int rr = row < rows ? row : 0, map = rr / kwmax, r = rr % kwmax;
+    const TapScale& t = set.s[map / kNumOri];
+    const bool act = row < rows && r < t.kW;
+    const float2* src = taps + (size_t)(map / kNumOri) * stride +
+                        ((size_t)(map % kNumOri) * t.kW + (act ? r : 0)) * t.kW;
+    float2 v[C::E];
+#pragma unroll
+    for (int e = 0; e < C::E; ++e) {
+        int c = in_index<N>(e, lane) + t.kX;
+        if (c >= N) c -= N;
+        v[e] = c < t.kW ? src[c] : make_float2(0.f, 0.f);
+    }
+    bimpdev::fft<N, false>(v, lds + grp * bimpdev::fft_lds_floats<N>(), lane, tw);
+    if (act) {
+        float2* p = out + (size_t)row * N;
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) p[out_index<N>(e, lane)] = v[e];
+    }
+}
+
+// Column transforms of those rows (zero elsewhere): the spectra Q_o and, for o = 0..4, the
+// quadrature bank G_o = Re Q_o / (FH*FW) of the detection path's inverse column pass, both
+// kx-major.  blockIdx.x: column block, .y: scale * 8 + orientation.
+template <int N>
+__global__ void __launch_bounds__(ACfg<N>::THREADS) k_bank_cols(const float2* __restrict__ in,
+                                                                TapSet set, int W, int kwmax,
+                                                                float invN,
+                                                                const float2* __restrict__ tw) {
+    using A = ACfg<N>;
+    extern __shared__ float2 lds2[];
+    const int j = blockIdx.y / kNumOri, o = blockIdx.y % kNumOri;
+    const TapScale& t = set.s[j];
+    const float2* src = in + (size_t)blockIdx.y * kwmax * W;
+    const int c0 = blockIdx.x * A::CB, b = threadIdx.x % A::CB, y0 = threadIdx.x / A::CB;
+    float2 v[A::E];
+#pragma unroll
+    for (int i = 0; i < A::E; ++i) {
+        int r = y0 + i * A::TPV + t.kX;
+        if (r >= N) r -= N;
+        v[i] = r < t.kW ? src[(size_t)r * W + c0 + b] : make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < A::E; ++i) lds2[b * A::S + y0 + i * A::TPV] = v[i];
+    __syncthreads();
+    const int g = group_of<A::TPV>(threadIdx.x), lane = threadIdx.x % A::TPV;
+    float2* my = lds2 + (size_t)g * A::S;
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) v[e] = my[in_index<N>(e, lane)];
+    bimpdev::stage_sync<A::TPV>();
+    bimpdev::fft<N, false>(v, reinterpret_cast<float*>(my), lane, tw);
+    pin<A::E>(v);
+    const size_t at = ((size_t)o * W + c0 + g) * N;
+#pragma unroll
+    for (int e = 0; e < A::E; ++e) {
+        const int ky = out_index<N>(e, lane);
+        t.Q[at + ky] = v[e];
+        if (o < kUniqueOri) t.G[at + ky] = v[e].x * invN;
+    }
 }
 
 // ---------------------------------------------------------------- backward pipeline
@@ -321,6 +445,7 @@ __global__ void __launch_bounds__(kRowThreads) k_z_rows(const float2* __restrict
 #pragma unroll
     for (int e = 0; e < C::E; ++e) v[e] = t[blk_at(in_index<N>(e, lane), y, Hc, sh)];
     bimpdev::fft<N, true>(v, lds + grp * bimpdev::fft_lds_floats<N>(), lane, tw);
+    pin<C::E>(v);
     if (act) {
         float2* z = Z + (size_t)row * N;
         float* c = Cm + (size_t)row * N;
@@ -553,6 +678,7 @@ __global__ void __launch_bounds__(ACfg<N>::THREADS) k_adj_cols(const float2* __r
         for (int e = 0; e < A::E; ++e) v[e] = my[in_index<N>(e, lane)];
         bimpdev::stage_sync<A::TPV>();
         bimpdev::fft<N, false>(v, reinterpret_cast<float*>(my), lane, tw);
+        pin<A::E>(v);
         const float2* q = set.Q[j] + ((size_t)o * W + kx) * N;
 #pragma unroll
         for (int e = 0; e < A::E; ++e) {
@@ -802,7 +928,8 @@ hipError_t diff_prepare(int n) {
 #define X(N)                                                                                 \
     if (n == N) {                                                                            \
         const std::pair<const void*, int> f[] = {                                            \
-            {(const void*)k_c2c_rows<N, false>, row_lds<N>()},                               \
+            {(const void*)k_bank_rows<N>, row_lds<N>()},                                     \
+            {(const void*)k_bank_cols<N>, ACfg<N>::LDS},                                     \
             {(const void*)k_pad_rows<N>, row_lds<N>()},                                      \
             {(const void*)k_z_rows<N>, row_lds<N>()},                                        \
             {(const void*)k_gz_rows<N>, row_lds<N>()},                                       \
@@ -823,11 +950,34 @@ hipError_t diff_prepare(int n) {
     return hipErrorInvalidValue;
 }
 
-hipError_t diff_rows(float2* data, int rows, int n, const float2* tw, hipStream_t s) {
+hipError_t diff_taps(const TapSet& set, const TapTrig& trig, float gamma, float2* taps,
+                     size_t stride, hipStream_t s) {
+    k_taps<<<dim3(kNumOri, set.n), kTapThreads, 0, s>>>(set, trig, gamma, taps, stride);
+    return hipGetLastError();
+}
+
+hipError_t diff_bank_rows(const TapSet& set, const float2* taps, size_t stride, int kwmax, int FW,
+                          float2* out, const float2* tw, hipStream_t s) {
+    const int rows = set.n * kNumOri * kwmax;
 #define X(N)                                                                                 \
-    if (n == N) {                                                                            \
-        k_c2c_rows<N, false><<<row_blocks<N>(rows), kRowThreads, row_lds<N>(), s>>>(data, rows, \
-                                                                                    tw);     \
+    if (FW == N) {                                                                           \
+        k_bank_rows<N><<<row_blocks<N>(rows), kRowThreads, row_lds<N>(), s>>>(               \
+            taps, stride, set, kwmax, rows, out, tw);                                        \
+        return hipGetLastError();                                                            \
+    }
+    BIMP_FOR_SIZES(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+
+hipError_t diff_bank_cols(const TapSet& set, const float2* in, int kwmax, int FH, int FW,
+                          float invN, const float2* tw, hipStream_t s) {
+#define X(N)                                                                                 \
+    if (FH == N) {                                                                           \
+        using A = ACfg<N>;                                                                   \
+        if (FW % A::CB) return hipErrorInvalidValue;                                         \
+        k_bank_cols<N><<<dim3(FW / A::CB, set.n * kNumOri), A::THREADS, A::LDS, s>>>(        \
+            in, set, FW, kwmax, invN, tw);                                                   \
         return hipGetLastError();                                                            \
     }
     BIMP_FOR_SIZES(X)
@@ -859,18 +1009,6 @@ hipError_t diff_pyr_down(const float* src, int sw, int sh, float* dst, int dw, i
 hipError_t diff_pyr_down_adj(const float* gdst, int dw, int dh, float* gsrc, int sw, int sh,
                              int nb, hipStream_t s) {
     k_pyr_down_adj<<<dim3((sw + 127) / 128, sh, nb), 128, 0, s>>>(gdst, dw, dh, gsrc, sw, sh);
-    return hipGetLastError();
-}
-
-hipError_t diff_q_to_g(const float2* Q, int FH, int FW, float invN, float* G, hipStream_t s) {
-    const size_t n = (size_t)kUniqueOri * FH * FW;
-    k_q_to_g<<<ew(n), 256, 0, s>>>(Q, n, invN, G);
-    return hipGetLastError();
-}
-
-hipError_t diff_bank_pad(const float* ke, const float* ko, int kW, int kX, int FH, int FW,
-                         float2* out, hipStream_t s) {
-    k_bank_pad<<<dim3((FW + 127) / 128, FH, kNumOri), 128, 0, s>>>(ke, ko, kW, kX, FH, FW, out);
     return hipGetLastError();
 }
 

@@ -50,9 +50,34 @@ struct AdjBuffers {
     uint2* gm;
 };
 
+// What the taps of a scale follow from, and where its bank goes.
+struct TapScale {
+    float lambda, fs, negInv;  // negInv: -1 / (2 sigma^2) as the FP32 taps use it
+    double sigma;              // FP64 sigma of the derivatives
+    int kW, kX;
+    float* dK;                 // 4 x 8 x kW x kW: dKe/dr, dKo/dr, dKe/dg, dKo/dg
+    float2* Q;                 // 8 x FW x FH
+    float* G;                  // 5 x FW x FH
+};
+struct TapSet {
+    int n;
+    TapScale s[kAdjMax];
+};
+// sine and cosine of the orientations, FP32 (of the FP32 angle) and FP64
+struct TapTrig {
+    float st[kNumOri], ct[kNumOri];
+    double std[kNumOri], ctd[kNumOri];
+};
+
 hipError_t diff_prepare(int n);
-// in-place forward transforms of contiguous rows
-hipError_t diff_rows(float2* data, int rows, int n, const float2* tw, hipStream_t s);
+// bank of the current parameters for one group of scales: taps and tap derivatives, row
+// transforms of the kwmax x FW tap rows per scale and orientation, then columns into Q and G
+hipError_t diff_taps(const TapSet& set, const TapTrig& trig, float gamma, float2* taps,
+                     size_t stride, hipStream_t s);
+hipError_t diff_bank_rows(const TapSet& set, const float2* taps, size_t stride, int kwmax, int FW,
+                          float2* out, const float2* tw, hipStream_t s);
+hipError_t diff_bank_cols(const TapSet& set, const float2* in, int kwmax, int FH, int FW,
+                          float invN, const float2* tw, hipStream_t s);
 // forward column transforms of H x W maps, clamp-padded to FH rows, into kx-major spectra
 hipError_t diff_cols_kx(const float2* in, int H, int FH, int W, const AdjInts& k, int nscales,
                         int maps, float2* out, const float2* tw, hipStream_t s);
@@ -60,9 +85,6 @@ hipError_t diff_pyr_down(const float* src, int sw, int sh, float* dst, int dw, i
                          hipStream_t s);
 hipError_t diff_pyr_down_adj(const float* gdst, int dw, int dh, float* gsrc, int sw, int sh,
                              int nb, hipStream_t s);
-hipError_t diff_q_to_g(const float2* Q, int FH, int FW, float invN, float* G, hipStream_t s);
-hipError_t diff_bank_pad(const float* ke, const float* ko, int kW, int kX, int FH, int FW,
-                         float2* out, hipStream_t s);
 // backward of one group, in order: padded row transforms into T (then diff_cols_kx from T
 // into D), Z's columns, Z's rows with the cells adjoint and gZ's rows, gZ's columns, then the
 // image rows into the level's gradient and the parameter partials

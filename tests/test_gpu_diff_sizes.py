@@ -65,3 +65,27 @@ def test_batch_equals_single_images(B, w, h, n):
         ps += p1
     # the library adds the images' partial sums one by one in double
     assert np.allclose(gp, ps, rtol=1e-9, atol=1e-9 * np.abs(ps).max())
+
+
+# 841, 1089 and 2809 taps: below, just above and above two of the chunks the sums walk
+@pytest.mark.parametrize("lam", [4.0, 4.6, 7.4])
+def test_bank_of_new_parameters(B, lam):
+    """Responses after a parameter change equal those of a context created with the parameters,
+    bit for bit, and the FP64 restatement's within the form's 1e-4."""
+    w, h, ratio, gamma = 130, 96, 0.61, 0.45
+    lams = np.array([lam], np.float32)
+    img = O.synth_frame(w, h, 12, 5).astype(np.float32)[None] / np.float32(255)
+    opt = B.default_options()
+    opt.sigma_ratio, opt.gamma = ratio, gamma
+    x = B.DeviceBuffer(img.nbytes)
+    x.upload(img)
+    got = []
+    for d in (B.Diff(w, h, lams), B.Diff(w, h, lams, opt)):
+        d.set_params(ratio, gamma)
+        out = B.DeviceBuffer(4 * d.response_size)
+        d.forward(x.ptr.value, 1, out.ptr.value)
+        got.append(out.download(np.zeros(d.response_size, np.float32)))
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    ref = np.concatenate([r.ravel() for r in DiffRef(w, h, lams).forward(
+        img[0].astype(np.float64), ratio=float(np.float32(ratio)), gamma=float(np.float32(gamma)))])
+    assert np.abs(got[0] - ref).max() <= 1e-4 * np.abs(ref).max()
