@@ -17,45 +17,44 @@
 namespace {
 
 // ------------------------------------------------------------------ colour histogram
-// One thread per keypoint (a window holds at most (2p)^2 pixels, p = (int)(log2(size)/2)).
-// The histogram arithmetic is the reference's: a channel byte is a signed char v, bin k
-// collects 31.875*k < v < 31.875*(k+1), so only bytes 1..127 count (bins 0..3); the counts
-// are scaled by 0.5 / (3 * pixels) in double.  Pixels outside the image are skipped (the
-// reference's inclusive bounds also read column `width` and row `height`).
+// One thread per keypoint and channel (a window holds at most (2p)^2 pixels, p =
+// (int)(log2(size)/2)).  The histogram arithmetic is the reference's: a channel byte is a signed
+// char v, bin k collects 31.875*k < v < 31.875*(k+1), so only bytes 1..127 count (bins 0..3); the
+// counts are scaled by 0.5 / (3 * pixels) in double.  Pixels outside the image are skipped (the
+// reference's inclusive bounds also read column `width` and row `height`).  Bound by the latency
+// of one thread's chain (logarithm, pixels, divisions): 4.9 us for 8000 keypoints, 7.0 us with
+// one thread for the three channels.
 __global__ void __launch_bounds__(64) k_color_features(const float* __restrict__ kp, int ld, int n,
                                                        const uint8_t* __restrict__ bgr,
                                                        size_t pitch, int width, int height,
                                                        float* __restrict__ desc, int desc_ld) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = e / 3, ch = e - 3 * i;
     if (i >= n) return;
     const float x = kp[i], y = kp[(size_t)ld + i], size = kp[4 * (size_t)ld + i];
     const int cx = (int)x, cy = (int)y;
     const int p = (int)(log2((double)size) / 2.0);
-    unsigned cnt[12] = {0};  // bins 0..3 of B, G, R (bins 4..7 cannot be reached)
+    unsigned cnt[4] = {0};  // bins 0..3 (bins 4..7 cannot be reached)
     int found = 0;
     for (int iy = cy - p; iy < cy + p; ++iy) {
         if (iy < 0 || iy >= height) continue;
-        const uint8_t* row = bgr + (size_t)iy * pitch;
+        const uint8_t* row = bgr + (size_t)iy * pitch + ch;
         for (int ix = cx - p; ix < cx + p; ++ix) {
             if (ix < 0 || ix >= width) continue;
             found += 3;
+            const int v = row[3 * ix];
+            // 31.875*k < v < 31.875*(k+1) for integer v in 1..127 is k = (8*v) / 255
+            const int bin = v >= 1 && v <= 127 ? (8 * v) / 255 : 4;
 #pragma unroll
-            for (int ch = 0; ch < 3; ++ch) {
-                const int v = row[3 * ix + ch];
-                // 31.875*k < v < 31.875*(k+1) for integer v in 1..127 is k = (8*v) / 255
-                if (v >= 1 && v <= 127) cnt[ch * 4 + (8 * v) / 255] += 1;
-            }
+            for (int k = 0; k < 4; ++k) cnt[k] += bin == k ? 1u : 0u;
         }
     }
-    float* d = desc + (size_t)i * desc_ld;
+    float* d = desc + (size_t)i * desc_ld + 8 * ch;
 #pragma unroll
-    for (int ch = 0; ch < 3; ++ch) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const double c = k < 4 ? (double)cnt[ch * 4 + k] : 0.0;
-            // (0.5 * c) / found, rounded once to float as the reference does
-            d[ch * 8 + k] = (float)((0.5 * c) / (found * 1.0));
-        }
+    for (int k = 0; k < 8; ++k) {
+        const double c = k < 4 ? (double)cnt[k < 4 ? k : 0] : 0.0;
+        // (0.5 * c) / found, rounded once to float as the reference does
+        d[k] = (float)((0.5 * c) / (found * 1.0));
     }
 }
 
@@ -338,8 +337,9 @@ int bimp_color_features(const float* d_kp, int ld, int n, const uint8_t* d_bgr, 
         width <= 0 || height <= 0 || bgr_pitch < (size_t)3 * width)
         return BIMP_E_ARG;
     if (n == 0) return BIMP_OK;
-    k_color_features<<<(n + 63) / 64, 64, 0, (hipStream_t)stream>>>(d_kp, ld, n, d_bgr, bgr_pitch,
-                                                                    width, height, d_desc, desc_ld);
+    const unsigned blocks = (unsigned)((3 * (long long)n + 63) / 64);
+    k_color_features<<<blocks, 64, 0, (hipStream_t)stream>>>(d_kp, ld, n, d_bgr, bgr_pitch, width,
+                                                             height, d_desc, desc_ld);
     return hipGetLastError() == hipSuccess ? BIMP_OK : BIMP_E_DEVICE;
 }
 

