@@ -109,6 +109,8 @@ void free_all(bimp_ctx* c) {
     (void)hipFree(c->T);
     (void)hipFree(c->R2);
     (void)hipFree(c->T2);
+    (void)hipFree(c->Rs);
+    (void)hipFree(c->Ts);
     if (c->frameExec) (void)hipGraphExecDestroy(c->frameExec);
     if (c->capStream) (void)hipStreamDestroy(c->capStream);
     if (c->side) (void)hipStreamDestroy(c->side);
@@ -193,6 +195,58 @@ int upload_frame(bimp_ctx* c, const uint8_t* img, size_t pitch, hipStream_t s) {
     return BIMP_OK;
 }
 
+// The groups of a small step: one launch per stage for all of them, then their cells.
+int run_small(bimp_ctx* c, const Step& st, const uint8_t* const* lv, const size_t* lp, bool cells,
+              hipStream_t q) {
+    bimpk::SmallJobs jobs;
+    jobs.n = st.small;
+    double bytes[4] = {};
+    int scales = 0;
+    for (int k = 0; k < st.small; ++k) {
+        const Group& gr = c->groups[st.index + k];
+        const Scale& s0 = c->sc[gr.first];
+        const auto& g = s0.g;
+        bimpk::SmallJob& j = jobs.j[k];
+        j.FW = g.FW;
+        j.FH = g.FH;
+        j.H = g.H;
+        j.W = g.W;
+        j.ldr = g.FW / 2 + 1;
+        j.Hc = s0.Hc;
+        j.Wc = s0.Wc;
+        j.ldc = s0.ldc;
+        j.img = lv[g.level];
+        j.pitch = lp[g.level];
+        j.R = c->Rs + gr.rOff;
+        j.T = c->Ts + gr.tOff;
+        j.rstride = (size_t)g.H * j.ldr;
+        j.tstride = (size_t)kNumOri * s0.Hc * g.FW;
+        j.twW = c->tw[g.FW];
+        j.twH = c->tw[g.FH];
+        j.ss.n = gr.n;
+        for (int i = 0; i < gr.n; ++i) {
+            const Scale& sk = c->sc[gr.first + i];
+            j.ss.kX[i] = sk.g.kX;
+            j.ss.G[i] = sk.G;
+            j.ss.DT[i] = sk.DT;
+            j.ss.C[i] = sk.C;
+        }
+        const double n = gr.n;
+        bytes[0] += n * ((double)g.H * g.W + 8.0 * g.H * j.ldr);
+        bytes[1] += n * (8.0 * g.H * j.ldr + 8.0 * j.ldr * g.FH);
+        bytes[2] += n * (8.0 * j.ldr * g.FH + 4.0 * kUniqueOri * g.FW * g.FH +
+                         8.0 * kNumOri * s0.Hc * g.FW);
+        bytes[3] += n * (8.0 * kNumOri * s0.Hc * g.FW + 4.0 * kNumOri * s0.Hc * s0.Wc);
+        scales += gr.n;
+    }
+    static const int fam[4] = {F_FWD_ROWS, F_FWD_COLS, F_INV_COLS, F_INV_ROWS};
+    for (int stage = 0; stage < 4; ++stage) {
+        LaunchScope ls(c, q, fam[stage], bytes[stage]);
+        HIPCHK(c, bimpk::launch_small_stage(jobs, stage, c->opt.input_scale, q));
+    }
+    return cells ? launch_cells_group(c, (size_t)c->groups[st.index].first, scales, q) : BIMP_OK;
+}
+
 // Parts of a frame for graph capture (run_filter's `part`): the whole frame as issued eagerly,
 // or, captured one per graph: the per-frame reset, the work on levels above 0 (pyramid
 // included), the level-0 work, or both of those in order on one stream.
@@ -261,6 +315,9 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
     for (const Step& st : c->steps)
         if ((st.direct ? c->sc[st.index].g.level : c->sc[c->groups[st.index].first].g.level) == 0)
             lastL0 = &st;
+    auto on_side = [&](const Step& st) {
+        return (st.direct ? c->sc[st.index].g.level : c->sc[c->groups[st.index].first].g.level) > 0;
+    };
     auto run_step = [&](const Step& st) -> int {
         if (st.direct) {
             const Scale& s0 = c->sc[st.index];
@@ -293,6 +350,7 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
             }
             return BIMP_OK;
         }
+        if (st.small) return run_small(c, st, lv, lp, cells, on_side(st) && useSide ? c->side : s);
         const Group& gr = c->groups[st.index];
         const auto& g = c->sc[gr.first].g;
         // groups above level 0 own R2/T2 whenever the context has a side stream, on s as well
@@ -374,9 +432,6 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
     };
     // Second-stream steps are issued first, so that the level-0 cells handed to that stream
     // below queue behind its own transforms rather than ahead of them.
-    auto on_side = [&](const Step& st) {
-        return (st.direct ? c->sc[st.index].g.level : c->sc[c->groups[st.index].first].g.level) > 0;
-    };
     for (int pass = useSide ? 0 : 1; pass < 2; ++pass) {
         for (const Step& st : c->steps) {
             if (useSide && on_side(st) != (pass == 0)) continue;
@@ -441,6 +496,35 @@ int run_keypoints(bimp_ctx* c, void* out, int cap, int matrix_ld, hipStream_t s)
     c->maxValid = false;
     c->slotsClean = true;
     return BIMP_OK;
+}
+
+// Turns the last steps of the frame, as far as they are FFT groups of transforms of at most 512
+// points (bimpk::small_size) whose T together stays in the last-level cache, into one step
+// whose stages are one launch each.  A frame with other level-0 work keeps its level-0 groups
+// apart, so that the rest still runs beside them.  Returns whether every step went into it.
+bool merge_small_groups(bimp_ctx* c) {
+    const size_t n = c->steps.size();
+    size_t k = n, t = 0;
+    auto level = [&](size_t i) { return c->sc[c->groups[c->steps[i].index].first].g.level; };
+    while (k > 0 && n - k < bimpk::kSmallJobs) {
+        const Step& st = c->steps[k - 1];
+        if (st.direct) break;
+        const Group& gr = c->groups[st.index];
+        const Scale& s0 = c->sc[gr.first];
+        const size_t bytes = (size_t)gr.n * kNumOri * s0.Hc * s0.g.FW * sizeof(float2);
+        if (!bimpk::small_size(s0.g.FW) || !bimpk::small_size(s0.g.FH) || t + bytes > kTBudgetBytes)
+            break;
+        t += bytes;
+        --k;
+    }
+    if (k > 0)
+        while (k < n && level(k) == 0) ++k;
+    if (n - k < 2) return false;
+    Step st = c->steps[k];
+    st.small = (int)(n - k);
+    c->steps.resize(k);
+    c->steps.push_back(st);
+    return k == 0;
 }
 
 int ensure_kp_buf(bimp_ctx* c, size_t bytes) {
@@ -791,7 +875,7 @@ int bimp_create(int width, int height, const float* lambdas, int n, const bimp_o
     // run_filter); then direct launches do not mix levels either.
     bool spans[2] = {false, false};
     for (const auto& s : c->sc) spans[s.g.level > 0 ? 1 : 0] = true;
-    const bool sideStream = spans[0] && spans[1] && !(c->opt.flags & BIMP_FLAG_SINGLE_STREAM);
+    bool sideStream = spans[0] && spans[1] && !(c->opt.flags & BIMP_FLAG_SINGLE_STREAM);
     bool prevFft = false;
     for (int i = 0; i < (int)c->sc.size(); ++i) {
         const auto& g = c->sc[i].g;
@@ -825,12 +909,24 @@ int bimp_create(int width, int height, const float* lambdas, int n, const bimp_o
         c->steps.push_back({false, (int)c->groups.size() - 1});
         prevFft = true;
     }
-    size_t rMax[2] = {0, 0}, tMax[2] = {0, 0};
+    if (merge_small_groups(c)) sideStream = false;
+    size_t rMax[2] = {0, 0}, tMax[2] = {0, 0}, rSmall = 0, tSmall = 0;
     std::vector<int> sizes;
     const unsigned hw = std::thread::hardware_concurrency();
     const int threads = (int)std::max(1u, std::min(16u, hw ? hw : 1u));
-    for (const auto& gr : c->groups) {
+    int smallFirst = (int)c->groups.size();
+    for (const Step& st : c->steps)
+        if (st.small) smallFirst = st.index;
+    for (int gi = 0; gi < (int)c->groups.size(); ++gi) {
+        Group& gr = c->groups[gi];
         const Scale& s0 = c->sc[gr.first];
+        if (gi >= smallFirst) {
+            gr.rOff = rSmall;
+            gr.tOff = tSmall;
+            rSmall += (size_t)gr.n * s0.g.H * (s0.g.FW / 2 + 1);
+            tSmall += (size_t)gr.n * kNumOri * s0.Hc * s0.g.FW;
+            continue;
+        }
         const int k = s0.g.level > 0 ? 1 : 0;
         rMax[k] = std::max(rMax[k], (size_t)gr.n * s0.g.H * (s0.g.FW / 2 + 1));
         const size_t ts = (size_t)kNumOri * s0.Hc * s0.g.FW;
@@ -897,7 +993,9 @@ int bimp_create(int width, int height, const float* lambdas, int n, const bimp_o
     if ((rMax[0] && dalloc(&c->R, rMax[0]) != hipSuccess) ||
         (tMax[0] && dalloc(&c->T, tMax[0]) != hipSuccess) ||
         (rMax[1] && dalloc(&c->R2, rMax[1]) != hipSuccess) ||
-        (tMax[1] && dalloc(&c->T2, tMax[1]) != hipSuccess))
+        (tMax[1] && dalloc(&c->T2, tMax[1]) != hipSuccess) ||
+        (rSmall && dalloc(&c->Rs, rSmall) != hipSuccess) ||
+        (tSmall && dalloc(&c->Ts, tSmall) != hipSuccess))
         return bail(BIMP_E_ALLOC, "scratch");
     // The fork, hand-off and join events order kernels of this device only, so they skip the
     // system-scope fence (the host sees results through the caller's stream, whose kernels

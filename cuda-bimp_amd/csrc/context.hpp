@@ -39,11 +39,12 @@ struct Scale {
     void* frag = nullptr;  // B-operand fragments of every tap block (16-bit taps)
 };
 
-// One step of a frame: an FFT resolution group or one direct-form scale.
+// One step of a frame: an FFT resolution group, several small groups, or direct-form scales.
 struct Step {
     bool direct;
-    int index;  // FFT: group index; direct: first scale
+    int index;  // FFT: (first) group index; direct: first scale
     int n = 1;  // direct: consecutive scales of one level in one launch
+    int small = 0;  // FFT: groups index .. index + small - 1 share each stage's launch
     bimpk::DirectJob* jobs = nullptr;  // direct: device job table
     int tiles = 0;
     size_t lds = 0;
@@ -52,6 +53,7 @@ struct Step {
 // Scales sharing pyramid level and transform size; each FFT stage runs once per group.
 struct Group {
     int first, n;
+    size_t rOff = 0, tOff = 0;  // small groups: their parts of Rs and Ts
 };
 
 struct ProfEv {
@@ -110,6 +112,9 @@ struct bimp_ctx {
     float2* R2 = nullptr;
     float2* T2 = nullptr;
     size_t tCap2 = 0;
+    // intermediates of the groups of a small step
+    float2* Rs = nullptr;
+    float2* Ts = nullptr;
     // this device's copy of the static keypoint staging of bimp_detect_u8_noalloc
     bimp_keypoint* noallocStaging = nullptr;
     // BIMP_FLAG_GRAPH: the frame as one executable graph, rebuilt when its frame or output

@@ -12,6 +12,7 @@
 //   k_nms_*        threshold, strict 8-neighbour max, parabola, ordered compaction (:714-743)
 #include <algorithm>
 #include <cmath>
+#include <utility>
 #include <vector>
 
 #include "fft_device.hpp"
@@ -469,6 +470,316 @@ __global__ void __launch_bounds__(InvRowCfg<FW>::THREADS) k_inv_rows_p(
                 if (x < Wc) out[x] = __builtin_amdgcn_sqrtf(v[e].x * v[e].x + v[e].y * v[e].y);
             }
         }
+    }
+}
+
+// ------------------------------------------------------------------ small groups together
+// The resolution groups of a small frame, or of the upper pyramid levels of a larger one, are
+// launch-bound: each stage of each group takes 4 to 10 us whatever its size, one after the
+// other.  Where two or more groups have transforms of at most 512 points, each stage of
+// all of them is one launch: a job per group, its workgroups numbered from block0[stage], the
+// transform length chosen per workgroup.  Same arithmetic as the kernels above, with twiddles
+// from global memory and no persistent loop.  A 320 x 240 frame with nine scales on five levels
+// goes from 33 launches to 13 and from 205 to 129 us, host to host; 1237 x 701 (three levels
+// together) from 603 to 580 us.  With 1024 points included, 640 x 480 (two groups of four
+// scales, already overlapped on two streams) went from 254 to 270 us, so the line is at 512.
+constexpr int kSmallRowThreads = 256, kSmallColThreads = 512;
+#define BIMP_SMALL_SIZES(X) X(16) X(32) X(64) X(128) X(256) X(512)
+
+// Row pairs of block `blk` of one scale, on the 64 lanes t of a wavefront whose LDS is `lds`.  As
+// k_fwd_rows.
+template <int FW>
+__device__ __forceinline__ void small_fwd_rows(const uint8_t* __restrict__ img, size_t pitch, int H,
+                                               int W, int kX, float scale, float2* __restrict__ R,
+                                               int ldr, const float2* __restrict__ tw, int blk,
+                                               int t, float* __restrict__ lds) {
+    using C = FFTCfg<FW>;
+    const int g = t / C::TPV, lane = t % C::TPV;
+    const int ya = 2 * (blk * RowCfg<FW>::VPB + g), yb = ya + 1;
+    const bool haveA = ya < H, haveB = yb < H;
+    float* my = lds + (size_t)g * 2 * FW;
+    const uint8_t* rowA = img + (size_t)(haveA ? ya : 0) * pitch;
+    const uint8_t* rowB = img + (size_t)(haveB ? yb : 0) * pitch;
+    // unconditional loads (rows clamped above) so that all of them are in flight at once
+    const float sa = haveA ? scale : 0.f, sb = haveB ? scale : 0.f;
+    float2 v[C::E];
+#pragma unroll
+    for (int e = 0; e < C::E; ++e) {
+        const int x = in_index<FW>(e, lane);
+        const int cx = x < W ? x : (x < W + kX ? W - 1 : 0);
+        v[e] = make_float2((float)rowA[cx] * sa, (float)rowB[cx] * sb);
+    }
+    fft<FW, false>(v, my, lane, tw);
+    float2* z = reinterpret_cast<float2*>(my);
+#pragma unroll
+    for (int e = 0; e < C::E; ++e) z[out_index<FW>(e, lane)] = v[e];
+    stage_sync<C::TPV>();
+    for (int k = lane; k <= FW / 2; k += C::TPV) {
+        const float2 z1 = z[k];
+        const float2 z2 = z[k == 0 ? 0 : FW - k];
+        if (haveA) R[(size_t)ya * ldr + k] = make_float2(0.5f * (z1.x + z2.x), 0.5f * (z1.y - z2.y));
+        if (haveB) R[(size_t)yb * ldr + k] = make_float2(0.5f * (z1.y + z2.y), -0.5f * (z1.x - z2.x));
+    }
+}
+
+// Row y of orientation map To into its complex-cell row `out`, on the TPV lanes of a group.
+// As k_inv_rows.
+template <int FW>
+__device__ __forceinline__ void small_inv_row(const float2* __restrict__ To, int Hc, int y,
+                                              bool active, int tsh, float* __restrict__ out, int Wc,
+                                              const float2* __restrict__ tw, int lane,
+                                              float* __restrict__ lds) {
+    using C = FFTCfg<FW>;
+    float2 v[C::E];
+    load_t_row<FW>(v, To, Hc, active ? y : 0, tsh, lane);
+    fft<FW, true, 8>(v, lds, lane, tw);
+    if (active) {
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) {
+            const int x = out_index<FW>(e, lane);
+            // native v_sqrt_f32 (1 ulp): the map tolerance is 1e-4 relative
+            if (x < Wc) out[x] = __builtin_amdgcn_sqrtf(v[e].x * v[e].x + v[e].y * v[e].y);
+        }
+    }
+}
+
+// The CB columns from kx0 of one scale, on the THREADS threads t whose LDS is lds2; every thread
+// of the workgroup calls it once (workgroup barriers).  As k_fwd_cols.
+template <int FH>
+__device__ __forceinline__ void small_fwd_cols(const float2* __restrict__ R, int ldr, int H, int kY,
+                                               float2* __restrict__ DT, int ncols,
+                                               const float2* __restrict__ tw, int kx0, int t,
+                                               float2* __restrict__ lds2) {
+    using C = FFTCfg<FH>;
+    using CC = ColCfg<FH>;
+    static_assert(CC::HALVES == 1 && FH * CC::CB / CC::THREADS <= 8, "one batch of loads");
+    const int g = t / C::TPV, lane = t % C::TPV;
+    float2* my = lds2 + (size_t)g * CC::S;
+    float2 v[C::E];
+    constexpr int YS = CC::THREADS / CC::CB, IT = FH * CC::CB / CC::THREADS;
+    const int b = t % CC::CB, y0 = t / CC::CB;
+    const bool in = kx0 + b < ncols;
+    float2 val[IT];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+        const int y = y0 + i * YS;
+        const int ry = y < H ? y : (y < H + kY ? H - 1 : 0);
+        val[i] = in ? R[(size_t)ry * ldr + kx0 + b] : make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < IT; ++i) lds2[b * CC::S + y0 + i * YS] = val[i];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < C::E; ++e) v[e] = my[in_index<FH>(e, lane)];
+    stage_sync<C::TPV>();
+    fft<FH, false>(v, reinterpret_cast<float*>(my), lane, tw);
+    const int kx = kx0 + g;
+    if (kx < ncols) {
+        float2* out = DT + (size_t)kx * FH;
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) out[out_index<FH>(e, lane)] = v[e];
+    }
+}
+
+// The pass (direct or partner) of orientation o over the column block at k0 of one scale, on the
+// THREADS threads t (group g, lane) whose LDS is lds2; every thread of the workgroup calls it
+// once (workgroup barriers), with `valid` false where there is nothing to do.  As one unit of
+// k_inv_cols.
+template <int FH>
+__device__ __forceinline__ void small_inv_cols(const float2* __restrict__ DT,
+                                               const float* __restrict__ G, int FW, int Hc, int o,
+                                               int partner, int k0, bool valid,
+                                               float2* __restrict__ To,
+                                               const float2* __restrict__ tw, int t, int g,
+                                               int lane, float2* __restrict__ lds2) {
+    using C = FFTCfg<FH>;
+    using IC = InvColCfg<FH>;
+    constexpr int CB = IC::CB;
+    const int half = FW / 2;
+    float* my = reinterpret_cast<float*>(lds2) + (size_t)g * fft_lds_floats<FH>();
+    const int og = o <= 4 ? o : kNumOri - o;
+    // direct: column kx = k0 + g; partner: stored column kx = k0 + 1 + g, output FW - kx
+    const int kx = k0 + partner + g;
+    const bool ok = valid && (partner ? (kx < half) : (kx <= half));
+    const float2* dcol = DT + (size_t)(ok ? kx : 0) * FH;
+    // bank column: direct o <= 4 -> kx, o >= 5 -> FW-kx; partner o <= 4 -> FW-kx, else kx
+    const int cg = ((o <= 4) != (partner != 0)) ? kx : (kx == 0 ? 0 : FW - kx);
+    const float* gcol = G + ((size_t)og * FW + (ok ? cg : 0)) * FH;
+    // D * G_o: per-lane base pointers, element offsets in_index(e, 0) known at compile
+    // time; the partner pass reads G at row FH - ky, except ky = 0 (lane 0 of e = 0)
+    float2 v[C::E];
+    const float2* dl = dcol + lane;
+    if (partner) {
+        const float* gl = gcol + (FH - lane);
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) {
+            const int ce = in_index<FH>(e, 0);
+            const float gv = e == 0 ? gcol[lane ? FH - lane : 0] : gl[-ce];
+            v[e] = cscale(dl[ce], gv);
+        }
+    } else {
+        const float* gl = gcol + lane;
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) {
+            const int ce = in_index<FH>(e, 0);
+            v[e] = cscale(dl[ce], gl[ce]);
+        }
+    }
+    fft<FH, true>(v, my, lane, tw);
+    if (partner) {
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) v[e].y = -v[e].y;
+    }
+    // output column of staging slot b: direct k0 + b; partner FW - (k0 + 1 + (CB-1-b))
+    const int slot = partner ? CB - 1 - g : g;
+    const int base = partner ? FW - k0 - CB : k0;
+#pragma unroll
+    for (int rq = 0; rq < IC::RL / IC::GB; ++rq) {
+        const int ylo = rq * IC::BRG;
+        if (ylo >= Hc) break;  // uniform
+        const int rows = min(Hc - ylo, IC::BRG);
+        __syncthreads();  // transforms and earlier readers of the region are done
+#pragma unroll
+        for (int m = 0; m < C::E / IC::RL; ++m)
+#pragma unroll
+            for (int gb = 0; gb < IC::GB; ++gb)
+                lds2[slot * IC::SS + gb * IC::BR + lane + C::TPV * m] =
+                        v[m * IC::RL + rq * IC::GB + gb];
+        __syncthreads();
+        // T is column-block-major: block base / CB holds rows 0..Hc-1 of its CB columns
+        // contiguously, so a unit's rows go out as one contiguous run
+        float2* const blk = To + (size_t)(base / CB) * Hc * CB;
+        for (int i = t; i < rows * CB; i += IC::THREADS) {
+            const int bt = i % CB, yy = i / CB;
+            const int ks = partner ? k0 + CB - bt : k0 + bt;  // stored column
+            const bool w = valid && (partner ? (ks < half) : (ks <= half));
+            if (w) blk[(size_t)(ylo + yy) * CB + bt] = lds2[bt * IC::SS + yy];
+        }
+    }
+}
+
+// (uniform: every thread of a workgroup finds the same job)
+__device__ __forceinline__ const SmallJob& small_job(const SmallJobs& jobs, int stage, int* b) {
+    int j = jobs.n - 1;
+    while (j > 0 && (int)blockIdx.x < jobs.j[j].block0[stage]) --j;
+    *b = (int)blockIdx.x - jobs.j[j].block0[stage];
+    return jobs.j[j];
+}
+
+// Column blocks of 512-thread workgroups: the shorter transforms put several blocks in one.
+template <int N>
+struct SmallCol {
+    static constexpr int THREADS = ColCfg<N>::THREADS, PER = kSmallColThreads / THREADS;
+    static_assert(PER * THREADS == kSmallColThreads, "whole blocks");
+    static constexpr size_t FWD = (size_t)ColCfg<N>::CB * ColCfg<N>::S * sizeof(float2);
+    static constexpr size_t INV = InvColCfg<N>::MAIN;
+};
+template <int N>
+constexpr size_t small_fwd_rows_lds() {
+    return (size_t)(kSmallRowThreads / FFTCfg<N>::TPV) * N * sizeof(float2);
+}
+template <int N>
+constexpr size_t small_inv_rows_lds() {
+    return (size_t)(kSmallRowThreads / FFTCfg<N>::TPV) * fft_lds_floats<N>() * sizeof(float);
+}
+
+__global__ void __launch_bounds__(kSmallRowThreads) k_small_fwd_rows(const SmallJobs jobs,
+                                                                     float scale) {
+    extern __shared__ float lds[];
+    int b;
+    const SmallJob& j = small_job(jobs, 0, &b);
+    switch (j.FW) {
+#define X(N)                                                                                 \
+    case N: {                                                                                \
+        /* one row block per wavefront; no workgroup barrier inside */                       \
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);                   \
+        const int nb = ((j.H + 1) / 2 + RowCfg<N>::VPB - 1) / RowCfg<N>::VPB;                \
+        const int u = b * (kSmallRowThreads / 64) + wave;                                    \
+        if (u >= nb * j.ss.n) return;                                                        \
+        const int sidx = u / nb;                                                             \
+        small_fwd_rows<N>(j.img, j.pitch, j.H, j.W, j.ss.kX[sidx], scale,                    \
+                          j.R + (size_t)sidx * j.rstride, j.ldr, j.twW, u % nb,              \
+                          threadIdx.x % 64, lds + wave * RowCfg<N>::VPB * 2 * N);            \
+        return;                                                                              \
+    }
+        BIMP_SMALL_SIZES(X)
+#undef X
+    }
+}
+
+__global__ void __launch_bounds__(kSmallColThreads) k_small_fwd_cols(const SmallJobs jobs) {
+    extern __shared__ float2 lds2[];
+    int b;
+    const SmallJob& j = small_job(jobs, 1, &b);
+    switch (j.FH) {
+#define X(N)                                                                                 \
+    case N: {                                                                                \
+        using S = SmallCol<N>;                                                               \
+        const int sub = threadIdx.x / S::THREADS;                                            \
+        const int nb = (j.ldr + ColCfg<N>::CB - 1) / ColCfg<N>::CB;                          \
+        const int u = b * S::PER + sub;                                                      \
+        const bool valid = u < nb * j.ss.n;                                                  \
+        const int sidx = valid ? u / nb : 0;                                                 \
+        /* columns past the last are neither read nor written */                             \
+        small_fwd_cols<N>(j.R + (size_t)sidx * j.rstride, j.ldr, j.H, j.ss.kX[sidx],         \
+                          j.ss.DT[sidx], j.ldr, j.twH, valid ? u % nb * ColCfg<N>::CB : j.ldr, \
+                          threadIdx.x % S::THREADS, lds2 + sub * (S::FWD / sizeof(float2))); \
+        return;                                                                              \
+    }
+        BIMP_SMALL_SIZES(X)
+#undef X
+    }
+}
+
+__global__ void __launch_bounds__(kSmallColThreads) k_small_inv_cols(const SmallJobs jobs) {
+    extern __shared__ float2 lds2[];
+    int b;
+    const SmallJob& j = small_job(jobs, 2, &b);
+    switch (j.FH) {
+#define X(N)                                                                                 \
+    case N: {                                                                                \
+        using S = SmallCol<N>;                                                               \
+        using C = FFTCfg<N>;                                                                 \
+        const int sub = threadIdx.x / S::THREADS, t = threadIdx.x % S::THREADS;              \
+        const int g = C::TPV == 64 ? __builtin_amdgcn_readfirstlane(t / 64) : t / C::TPV;    \
+        const int nblk = (j.FW / 2 + ColCfg<N>::CB) / ColCfg<N>::CB;                         \
+        /* unit: orientation fastest, then the pass, the column block and the scale */       \
+        const int u = b * S::PER + sub, o = u % kNumOri, partner = u / kNumOri % 2;          \
+        const int gcb = u / (2 * kNumOri);                                                   \
+        const bool valid = gcb < nblk * j.ss.n;                                              \
+        const int sidx = valid ? gcb / nblk : 0;                                             \
+        small_inv_cols<N>(j.ss.DT[sidx], j.ss.G[sidx], j.FW, j.Hc, o, partner,                \
+                         (valid ? gcb % nblk : 0) * ColCfg<N>::CB, valid,                    \
+                         j.T + (size_t)sidx * j.tstride + (size_t)o * j.Hc * j.FW, j.twH, t, g, \
+                         t % C::TPV, lds2 + sub * (S::INV / sizeof(float2)));                \
+        return;                                                                              \
+    }
+        BIMP_SMALL_SIZES(X)
+#undef X
+    }
+}
+
+__global__ void __launch_bounds__(kSmallRowThreads) k_small_inv_rows(const SmallJobs jobs) {
+    extern __shared__ float lds[];
+    int b;
+    const SmallJob& j = small_job(jobs, 3, &b);
+    switch (j.FW) {
+#define X(N)                                                                                 \
+    case N: {                                                                                \
+        using C = FFTCfg<N>;                                                                 \
+        constexpr int RPW = kSmallRowThreads / C::TPV;                                       \
+        const int g = C::TPV == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 64)        \
+                                   : threadIdx.x / C::TPV;                                   \
+        /* a workgroup's rows lie in one orientation map */                                  \
+        const int nrb = (j.Hc + RPW - 1) / RPW;                                              \
+        const int y = b % nrb * RPW + g, o = b / nrb % kNumOri, sidx = b / nrb / kNumOri;    \
+        small_inv_row<N>(j.T + (size_t)sidx * j.tstride + (size_t)o * j.Hc * j.FW, j.Hc, y, y < j.Hc, \
+                   j.tsh, j.ss.C[sidx] + ((size_t)o * j.Hc + y) * j.ldc, j.Wc, j.twW,        \
+                   threadIdx.x % C::TPV, lds + (size_t)g * fft_lds_floats<N>());             \
+        return;                                                                              \
+    }
+        BIMP_SMALL_SIZES(X)
+#undef X
     }
 }
 
@@ -1235,6 +1546,10 @@ static hipError_t prepare_n() {
 
 hipError_t prepare_common() {
     hipError_t e = hipSuccess;
+    for (const void* f : {(const void*)k_small_fwd_rows, (const void*)k_small_fwd_cols,
+                          (const void*)k_small_inv_cols, (const void*)k_small_inv_rows})
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
 #define X(HS)                                                                                \
     if (e == hipSuccess)                                                                     \
         e = hipFuncSetAttribute((const void*)k_cells<HS>,                                    \
@@ -1355,6 +1670,64 @@ hipError_t launch_inv_rows(int FW, int FH, const ScaleSet& ss, const float2* T, 
     BIMP_FOR_SIZES(X)
 #undef X
     return hipErrorInvalidValue;
+}
+
+bool small_size(int n) {
+#define X(N) if (n == N) return true;
+    BIMP_SMALL_SIZES(X)
+#undef X
+    return false;
+}
+
+// Workgroups of a job per stage, and the dynamic LDS of a workgroup: {blocks, bytes}.
+static std::pair<int, size_t> small_stage(const SmallJob& j, int stage) {
+    const int n = j.ss.n;
+    auto up = [](int a, int b) { return (a + b - 1) / b; };
+#define X(N)                                                                                 \
+    if (j.FW == N && stage == 0)                                                             \
+        return {up(up((j.H + 1) / 2, RowCfg<N>::VPB) * n, kSmallRowThreads / 64),            \
+                small_fwd_rows_lds<N>()};                                                    \
+    if (j.FH == N && stage == 1)                                                             \
+        return {up(up(j.ldr, ColCfg<N>::CB) * n, SmallCol<N>::PER),                          \
+                SmallCol<N>::FWD * SmallCol<N>::PER};                                        \
+    if (j.FH == N && stage == 2)                                                             \
+        return {up((j.FW / 2 + ColCfg<N>::CB) / ColCfg<N>::CB * n * 2 * kNumOri,             \
+                   SmallCol<N>::PER),                                                        \
+                SmallCol<N>::INV * SmallCol<N>::PER};                                        \
+    if (j.FW == N && stage == 3)                                                             \
+        return {up(j.Hc, kSmallRowThreads / FFTCfg<N>::TPV) * kNumOri * n,                   \
+                small_inv_rows_lds<N>()};
+    BIMP_SMALL_SIZES(X)
+#undef X
+    return {0, 0};
+}
+
+hipError_t launch_small_stage(SmallJobs& jobs, int stage, float scale, hipStream_t s) {
+    int blocks = 0;
+    size_t lds = 0;
+    if (jobs.n < 1 || jobs.n > kSmallJobs) return hipErrorInvalidValue;
+    for (int k = 0; k < jobs.n; ++k) {
+        SmallJob& j = jobs.j[k];
+        const int cb = col_batch(j.FH);
+        j.tsh = 0;
+        while ((1 << j.tsh) < cb) ++j.tsh;
+        if (!small_size(j.FW) || !small_size(j.FH) || j.FW % cb || (1 << j.tsh) != cb ||
+            j.Hc > j.FH)
+            return hipErrorInvalidValue;
+        const auto st = small_stage(j, stage);
+        j.block0[stage] = blocks;
+        blocks += st.first;
+        lds = std::max(lds, st.second);
+    }
+    if (stage == 0)
+        k_small_fwd_rows<<<blocks, kSmallRowThreads, lds, s>>>(jobs, scale);
+    else if (stage == 1)
+        k_small_fwd_cols<<<blocks, kSmallColThreads, lds, s>>>(jobs);
+    else if (stage == 2)
+        k_small_inv_cols<<<blocks, kSmallColThreads, lds, s>>>(jobs);
+    else
+        k_small_inv_rows<<<blocks, kSmallRowThreads, lds, s>>>(jobs);
+    return hipGetLastError();
 }
 
 template <int HS>

@@ -21,6 +21,27 @@ struct ScaleSet {
     float* C[kMaxBatch];
 };
 
+// A resolution group whose stages run in one launch each with those of other groups (all
+// transforms of at most 512 points).
+constexpr int kSmallJobs = 8;
+struct SmallJob {
+    int FW, FH, H, W;
+    int ldr;            // columns of the half spectrum, FW / 2 + 1
+    int Hc, Wc, ldc;    // complex-cell region and pitch
+    int tsh;            // log2 of the column blocks of T (set by the launch)
+    int block0[4];      // first workgroup of the job in each stage's launch (set by the launch)
+    const uint8_t* img;
+    size_t pitch;
+    float2 *R, *T;      // the group's own intermediates
+    size_t rstride, tstride;
+    const float2 *twW, *twH;
+    ScaleSet ss;
+};
+struct SmallJobs {
+    SmallJob j[kSmallJobs];
+    int n;
+};
+
 // Per-scale constants of the end-stop / inhibition stencil (host-derived).
 struct CellParams {
     int ea[kNumOri], eb[kNumOri];  // end-stop offsets (rows, cols)
@@ -121,12 +142,15 @@ hipError_t launch_inv_cols(int FH, const ScaleSet& ss, int FW, int Hc, float2* T
                            size_t tstride, const float2* tw, hipStream_t s);
 hipError_t launch_inv_rows(int FW, int FH, const ScaleSet& ss, const float2* T, size_t tstride,
                            int Hc, int Wc, int ldc, const float2* tw, hipStream_t s);
+// Stage 0..3 (forward rows, forward columns, inverse columns, inverse rows) of every job.
+bool small_size(int n);
+hipError_t launch_small_stage(SmallJobs& jobs, int stage, float scale, hipStream_t s);
 hipError_t launch_cells(const float* C, int Hc, int ldc, int FH, int FW, int H, int W,
                         const CellParams& p, float* Dm, float* Sm, unsigned* maxslot,
                         hipStream_t s);
 // End-stop/inhibition of up to kCellMaxScales scales in one launch (the arguments of
 // launch_cells per scale).
-constexpr int kCellMaxScales = 8;
+constexpr int kCellMaxScales = 12;  // (the job table of a launch is a kernel argument: < 4 KB)
 struct CellScale {
     const float* C;
     int Hc, ldc, FH, FW, H, W;
