@@ -1751,11 +1751,15 @@ static void make_cell_job(const MapView& mv, int FH, int FW, int H, int W, const
     auto first = [](int hh, int t) { return (hh + t - 1) / t; };
     auto end = [](int lim, int t) { return lim >= 0 ? lim / t + 1 : 0; };  // x0 <= lim
     tg.ix0 = first(HS, kCellTW);
-    tg.ix1 = std::max(tg.ix0, std::min(tg.tiles_x, end(W - HS - (kCellTW - 1), kCellTW)));
+    // (where the transform is as wide or high as the data, column W or row H would wrap around:
+    // the staged tile then ends one earlier; 1024 x 1024, eight scales: 108 us a frame against 160
+    // with every tile on the checked path)
+    const int wx = W >= FW ? 1 : 0, wy = H >= FH ? 1 : 0;
+    tg.ix1 = std::max(tg.ix0, std::min(tg.tiles_x, end(W - wx - HS - (kCellTW - 1), kCellTW)));
     tg.iy0 = first(HS, kCellTH);
-    tg.iy1 = std::max(tg.iy0, std::min(tg.tiles_y, end(H - HS - (kCellTH - 1), kCellTH)));
+    tg.iy1 = std::max(tg.iy0, std::min(tg.tiles_y, end(H - wy - HS - (kCellTH - 1), kCellTH)));
     // (interior staging offsets span 5 maps from the pair's base: 8 maps must fit 32 bits)
-    if (W >= FW || H >= FH || tg.ix0 >= tg.tiles_x || tg.iy0 >= tg.tiles_y ||
+    if (tg.ix0 >= tg.tiles_x || tg.iy0 >= tg.tiles_y ||
         (size_t)kNumOri * mv.Hc * mv.ldc * sizeof(float) > 0xffffffffu)
         tg.ix0 = tg.ix1 = tg.iy0 = tg.iy1 = 0;  // everything takes the checked path
     const int nin = (tg.ix1 - tg.ix0) * (tg.iy1 - tg.iy0);
