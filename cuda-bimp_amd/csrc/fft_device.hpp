@@ -330,15 +330,16 @@ struct LdsTw {
 // the exchanges.
 typedef const __attribute__((address_space(1))) float2* GlobalTw;
 
-template <int N, bool INV, int Ns, int R, class TW>
+// PERM: the stage follows an in-register exchange (kRegFirst), so that its butterfly m on a
+// lane is j = (lane % 8) * Ns + 8 m + lane / 8.
+template <int N, bool INV, int Ns, int R, bool PERM, class TW>
 __device__ __forceinline__ void butterflies(float2 (&v)[FFTCfg<N>::E], int lane, TW tw) {
     using C = FFTCfg<N>;
     constexpr int P = tw_row(R);
 #pragma unroll
     for (int m = 0; m < C::E / R; ++m) {
         if constexpr (Ns > 1) {
-            const int j = lane + C::TPV * m;
-            const int k = j % Ns;
+            const int k = PERM ? 8 * m + (lane >> 3) : (lane + C::TPV * m) % Ns;
             float4 t[P / 2];
             if constexpr (std::is_same<TW, LdsTw>::value) {
 #pragma unroll
@@ -380,8 +381,9 @@ __device__ __forceinline__ void butterflies(float2 (&v)[FFTCfg<N>::E], int lane,
 template <int Ns, int R, int VMAX>
 inline constexpr bool kVecFirst = Ns == 1 && R % 4 == 0 && (R <= VMAX || R > 16);
 
+// (64 lanes: room for the eight padded runs of the exchange after an in-register one)
 template <int N>
-__host__ __device__ constexpr int fft_lds_floats() { return N; }
+__host__ __device__ constexpr int fft_lds_floats() { return FFTCfg<N>::TPV == 64 ? N + 64 : N; }
 template <int Ns, int R, int VMAX>
 __device__ __forceinline__ int lds_pad(int i) {
     if constexpr (Ns == 1 && !kVecFirst<Ns, R, VMAX>)
@@ -453,23 +455,134 @@ __device__ __forceinline__ void exchange(float2 (&v)[FFTCfg<N>::E], float* lds, 
     stage_sync<C::TPV>();
 }
 
-template <int N, bool INV, int Ns, class L, int VMAX>
+// In-register first exchange.  With N = R1 R2 8 on 64 lanes, lane (a, l), a = lane / 8, l =
+// lane % 8, holds after the first stage the outputs r = 8 m' + t of its butterflies j = lane +
+// 64 m, elements j R1 + r; the second stage's leg j / 8 = a + 8 m of butterfly l R1 + r.  So
+// for each (m, m') an 8 x 8 transpose between the lane bits a and the register bits t puts
+// every element where a second-stage butterfly can use it, with no LDS and no wait: two bits by
+// the half-wave and row swaps, one instruction per register pair, the third by two row
+// rotations.  The second exchange then writes runs of N/8 elements, one per l, padded to N/8 + 8
+// so that the 64 lanes hit 64 banks.  The transforms' kernels wait on instruction latency, LDS
+// included, more than on bytes: with the first exchange in LDS as well, k_inv_cols<2560> took
+// 1168 us per 3840 x 2160 frame against 1042, k_inv_cols<1536> 283 us per 1920 x 1080 frame
+// against 274 and k_inv_rows<2048> 200 against 195.  (1024 = 16 16 4 does not have the form;
+// 4096 points span two wavefronts.)
+template <int N, int R1, int R2>
+inline constexpr bool kRegFirst = FFTCfg<N>::TPV == 64 && N == R1 * R2 * 8 && R1 % 8 == 0 &&
+                                  R2 == 8 * (FFTCfg<N>::E / R1);
+
+__device__ __forceinline__ void swap_lane_bit5(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                    false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_lane_bit4(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                    false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_lane_bit3(float& a, float& b) {
+    constexpr int kRor8 = 0x128;  // DPP row rotation by 8 lanes
+    const int x = __float_as_int(a), y = __float_as_int(b);
+    a = __int_as_float(__builtin_amdgcn_update_dpp(x, y, kRor8, 0xf, 0xc, false));
+    b = __int_as_float(__builtin_amdgcn_update_dpp(y, x, kRor8, 0xf, 0x3, false));
+}
+// Transposes lane bits 5..3 with the register index of x[8].
+__device__ __forceinline__ void transpose8(float (&x)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) swap_lane_bit5(x[i], x[i + 4]);
+#pragma unroll
+    for (int i = 0; i < 8; i += 4) {
+        swap_lane_bit4(x[i], x[i + 2]);
+        swap_lane_bit4(x[i + 1], x[i + 3]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) swap_lane_bit3(x[i], x[i + 1]);
+}
+template <int N, int R1, int R2>
+__device__ __forceinline__ void exchange_reg(float2 (&v)[FFTCfg<N>::E]) {
+    constexpr int M = FFTCfg<N>::E / R1, MP = R1 / 8;
+    float2 w[FFTCfg<N>::E];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int mp = 0; mp < MP; ++mp) {
+            float re[8], im[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                re[t] = v[m * R1 + 8 * mp + t].x;
+                im[t] = v[m * R1 + 8 * mp + t].y;
+            }
+            transpose8(re);
+            transpose8(im);
+#pragma unroll
+            for (int a = 0; a < 8; ++a) w[mp * R2 + a + 8 * m] = make_float2(re[a], im[a]);
+        }
+#pragma unroll
+    for (int e = 0; e < FFTCfg<N>::E; ++e) v[e] = w[e];
+}
+// The exchange after it, real parts then imaginary parts through LDS: run l of N/8 elements from
+// l (N/8 + 8).
+template <int N, int R1, int R2>
+__device__ __forceinline__ void exchange_padded(float2 (&v)[FFTCfg<N>::E], float* lds, int lane) {
+    using C = FFTCfg<N>;
+    constexpr int RUN = N / 8 + 8;
+    float* const out = lds + (lane & 7) * RUN + (lane >> 3);
+    const float* const in = lds + lane;
+#pragma unroll
+    for (int m = 0; m < C::E / R2; ++m)
+#pragma unroll
+        for (int r = 0; r < R2; ++r) out[8 * m + r * R1] = v[m * R2 + r].x;
+    stage_sync<C::TPV>();
+    float im[C::E];
+#pragma unroll
+    for (int e = 0; e < C::E; ++e) im[e] = v[e].y;
+#pragma unroll
+    for (int m = 0; m < C::E / 8; ++m)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) v[m * 8 + r].x = in[C::TPV * m + r * RUN];
+    stage_sync<C::TPV>();
+#pragma unroll
+    for (int m = 0; m < C::E / R2; ++m)
+#pragma unroll
+        for (int r = 0; r < R2; ++r) out[8 * m + r * R1] = im[m * R2 + r];
+    stage_sync<C::TPV>();
+#pragma unroll
+    for (int m = 0; m < C::E / 8; ++m)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) v[m * 8 + r].y = in[C::TPV * m + r * RUN];
+    stage_sync<C::TPV>();
+}
+
+template <int N, bool INV, int Ns, class L, int VMAX, int RP = 0>
 struct Stages;
-template <int N, bool INV, int Ns, int R, int... Rest, int VMAX>
-struct Stages<N, INV, Ns, RadList<R, Rest...>, VMAX> {
-    // tw points at this stage's rows (unused for the first stage)
+template <int N, bool INV, int Ns, int R, int... Rest, int VMAX, int RP>
+struct Stages<N, INV, Ns, RadList<R, Rest...>, VMAX, RP> {
+    // tw points at this stage's rows (unused for the first stage); RP: the radix of the stage
+    // before, if its exchange stayed in registers
     template <class TW>
     static __device__ __forceinline__ void run(float2 (&v)[FFTCfg<N>::E], float* lds, int lane,
                                                TW tw) {
-        butterflies<N, INV, Ns, R>(v, lane, tw);
+        butterflies<N, INV, Ns, R, (RP > 0)>(v, lane, tw);
         if constexpr (sizeof...(Rest) > 0) {
-            exchange<N, Ns, R, RadInfo<RadList<Rest...>>::first, VMAX>(v, lds, lane);
+            constexpr int R2 = RadInfo<RadList<Rest...>>::first;
+            constexpr bool reg = Ns == 1 && kRegFirst<N, R, R2>;
+            if constexpr (reg)
+                exchange_reg<N, R, R2>(v);
+            else if constexpr (RP > 0)
+                exchange_padded<N, RP, R>(v, lds, lane);
+            else
+                exchange<N, Ns, R, R2, VMAX>(v, lds, lane);
             constexpr int next_ns = Ns * R;
             constexpr int adv = Ns > 1 ? Ns * tw_row(R) : 0;  // float2
             if constexpr (std::is_same<TW, LdsTw>::value)
-                Stages<N, INV, next_ns, RadList<Rest...>, VMAX>::run(v, lds, lane, LdsTw{tw.p + adv / 2});
+                Stages<N, INV, next_ns, RadList<Rest...>, VMAX, reg ? R : 0>::run(
+                    v, lds, lane, LdsTw{tw.p + adv / 2});
             else
-                Stages<N, INV, next_ns, RadList<Rest...>, VMAX>::run(v, lds, lane, tw + adv);
+                Stages<N, INV, next_ns, RadList<Rest...>, VMAX, reg ? R : 0>::run(v, lds, lane,
+                                                                                   tw + adv);
         }
     }
 };

@@ -123,7 +123,9 @@ struct ColCfg {
     static constexpr int HALVES = (size_t)CB * (N + 2) * sizeof(float2) > 64u * 1024u ? 2 : 1;
     // column stride (complex): 2 (mod 16) puts the 8 columns of a 16-lane access 4 banks
     // apart, so staging writes (column index fastest) do not collide
-    static constexpr int S = N / HALVES + 2;
+    // (and room for the transform's exchange region)
+    static constexpr int S = N / HALVES + (HALVES == 2 && TPV == 64 ? 34 : 2);
+    static_assert(2 * S >= fft_lds_floats<N>(), "the exchange fits the column's staging");
 };
 
 // Column FFT of the row spectra R (H rows, ldr complex per row) with clamp padding in y:
