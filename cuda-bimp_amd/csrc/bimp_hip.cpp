@@ -296,19 +296,18 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
     lv[0] = src0;
     lp[0] = pitch0;
     for (int l = 1; l <= c->maxLevel; ++l) {
-        if (part == kPartLevel0) {  // the pyramid belongs to the upper-level part
-            lv[l] = c->level[l];
-            lp[l] = (size_t)c->levelW[l];
-            continue;
-        }
-        LaunchScope ls(c, pq, F_PYR,
-                       (double)c->levelW[l - 1] * c->levelH[l - 1] + (double)c->levelW[l] * c->levelH[l]);
-        HIPCHK(c, bimpk::launch_pyr_down(lv[l - 1], c->levelW[l - 1], c->levelH[l - 1], lp[l - 1],
-                                         c->level[l], c->levelW[l], c->levelH[l],
-                                         (size_t)c->levelW[l],
-                                         (c->opt.flags & BIMP_FLAG_RESIZE_CPU) != 0, pq));
         lv[l] = c->level[l];
         lp[l] = (size_t)c->levelW[l];
+    }
+    // the pyramid belongs to the upper-level part
+    for (int l = 0; l < c->maxLevel && part != kPartLevel0; l += bimpk::kPyrLevels) {
+        const int n = std::min(bimpk::kPyrLevels, c->maxLevel - l);
+        double bytes = (double)c->levelW[l] * c->levelH[l];
+        for (int k = 1; k <= n; ++k) bytes += (double)c->levelW[l + k] * c->levelH[l + k];
+        LaunchScope ls(c, pq, F_PYR, bytes);
+        HIPCHK(c, bimpk::launch_pyr_down(lv[l], lp[l], &c->level[l + 1], &c->levelW[l],
+                                         &c->levelH[l], n,
+                                         (c->opt.flags & BIMP_FLAG_RESIZE_CPU) != 0, pq));
     }
     // the last step at pyramid level 0: the frame's final transforms on s
     const Step* lastL0 = nullptr;

@@ -25,17 +25,15 @@ namespace bimpk {
 namespace {
 
 // ------------------------------------------------------------------ pyramid
+// reflect-101 of an index up to two outside [0, n); further out, some index inside
 __device__ __forceinline__ int reflect101(int i, int n) {
-    if (n == 1) return 0;
-    for (int it = 0; it < 4 && (i < 0 || i >= n); ++it) {
-        if (i < 0) i = -i;
-        if (i >= n) i = 2 * (n - 1) - i;
-    }
-    return i;
+    i = abs(i);
+    i = abs(i >= n ? 2 * (n - 1) - i : i);
+    return min(i, n - 1);
 }
 
-// 5x5 binomial [1 4 6 4 1]^2 / 256, reflect-101 border.  Round half to even: the float sum is
-// exact, so this equals OpenCV-CUDA pyrDown's saturate_cast of its FP32 sum
+// One pyramid level: 5x5 binomial [1 4 6 4 1]^2 / 256, reflect-101 border.  Round half to even:
+// the sum S is exact, so this equals OpenCV-CUDA pyrDown's saturate_cast of its FP32 sum
 // (cuda_bimp.cu:476).  half_up: (S + 128) >> 8, the fixed-point rounding of OpenCV's host
 // pyrDown, which the reference's resize_cpu option uses (cuda_bimp.cu:660-665).
 __global__ void k_pyr_down(const uint8_t* __restrict__ src, int sw, int sh, size_t spitch,
@@ -56,6 +54,149 @@ __global__ void k_pyr_down(const uint8_t* __restrict__ src, int sw, int sh, size
     }
     dst[(size_t)y * dpitch + x] =
         half_up ? (uint8_t)((acc + 128) >> 8) : (uint8_t)rintf((float)acc * (1.0f / 256.0f));
+}
+
+// Two to four levels of one frame in one launch, each from the one before, as above.  A
+// workgroup takes a tile of the last level, computes what that tile reads of every level below
+// it in LDS, and writes its own share of each.  It works on pixel pairs in 16-bit halves
+// (S <= 65280), rows first, so a pair costs two LDS words and a few integer operations per
+// pass.  A launch lasts about 4 us whatever it does, and a level waits for the one before:
+// 467 x 350 with four levels took 25 us in four launches of the kernel above and takes 14 in
+// one, 3840 x 2160 with four 53 and 38.  256 and 1024 threads: 19 and 13 us at 467 x 350, 43 and
+// 51 at 3840 x 2160.  A single level gains nothing worth having here (1920 x 1080: 12.0 and 9.3
+// us, 640 x 480: 6.5 and 6.9), and the kernel above, with two wavefronts and no LDS, fits
+// beside another stream's: the 1920 x 1080 precision form went from 517-528 to 516-530 us with
+// its single level on tiles.
+struct PyrJob {
+    const uint8_t* src;
+    size_t spitch;
+    uint8_t* dst[kPyrLevels];  // level i + 1 of the job, row pitch = its width
+    int w[kPyrLevels + 1], h[kPyrLevels + 1];
+    int n, tile, half_up;
+    int rows, pairs;  // source rows and level-1 pixel pairs per row that a tile reaches back to
+};
+constexpr int kPyrThreads = 512;
+
+__device__ __forceinline__ unsigned pyr_round(unsigned acc, int half_up) {
+    // two 16-bit sums to two bytes (bits 0-7 and 16-23)
+    const unsigned odd = (acc >> 8) & 0x00010001u;
+    return ((acc + (half_up ? 0x00800080u : 0x007f007fu + odd)) >> 8) & 0x00ff00ffu;
+}
+
+__global__ void __launch_bounds__(kPyrThreads) k_pyr_levels(PyrJob j) {
+    extern __shared__ unsigned px[];  // bytes of the level read, j.pairs + 1 words per row
+    const int pw = j.pairs + 1;
+    unsigned* const hs = px + j.rows * pw;  // its row sums, a pixel pair per word
+    // columns [xl, xh) and rows [yl, yh) of each level that the tile needs; xl is even
+    int xl[kPyrLevels + 1], xh[kPyrLevels + 1], yl[kPyrLevels + 1], yh[kPyrLevels + 1];
+    const int n = j.n, T = j.tile, tx = blockIdx.x, ty = blockIdx.y, tid = threadIdx.x;
+#pragma unroll
+    for (int i = kPyrLevels; i >= 0; --i) {
+        if (i > n) continue;
+        if (i == n) {
+            xl[i] = tx * T;
+            xh[i] = min(j.w[i], xl[i] + T);
+            yl[i] = ty * T;
+            yh[i] = min(j.h[i], yl[i] + T);
+        } else {
+            xl[i] = max(0, 2 * xl[i + 1] - 2);
+            xh[i] = min(j.w[i], 2 * xh[i + 1] + 1);
+            yl[i] = max(0, 2 * yl[i + 1] - 2);
+            yh[i] = min(j.h[i], 2 * yh[i + 1] + 1);
+        }
+    }
+    // Words of a level's row in px: the first byte is column 2 xl - 2 of the level above it, so
+    // the pair (x, x + 1) reads the words (x - xl) / 2 and the next.  Columns beyond the level
+    // hold the reflected ones.
+    {
+        const int words = (xh[1] - xl[1] + 1) / 2 + 1, ox = 2 * xl[1] - 2, w = j.w[0];
+        const int lw = words <= 16 ? 16 : words <= 32 ? 32 : 64, c = tid % lw;
+        const int x = ox + 4 * c, step = kPyrThreads / lw;
+        const bool inside = x >= 0 && x + 4 <= w;
+        int xr[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xr[k] = reflect101(x + k, w);
+        if (c < words)
+            for (int y = yl[0] + tid / lw; y < yh[0]; y += 4 * step) {
+                unsigned v[4];  // four rows in flight
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint8_t* row = j.src + (size_t)min(y + r * step, yh[0] - 1) * j.spitch;
+                    if (inside)
+                        __builtin_memcpy(&v[r], row + x, 4);
+                    else
+                        v[r] = row[xr[0]] | row[xr[1]] << 8 | row[xr[2]] << 16 |
+                               (unsigned)row[xr[3]] << 24;
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (y + r * step < yh[0]) px[(y + r * step - yl[0]) * pw + c] = v[r];
+            }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 1; i <= kPyrLevels; ++i) {
+        if (i > n) break;  // uniform
+        const int pairs = (xh[i] - xl[i] + 1) / 2;
+        {
+            const int lw = pairs <= 16 ? 16 : pairs <= 32 ? 32 : 64, c = tid % lw;
+            const int rows = yh[i - 1] - yl[i - 1];
+            if (c < pairs)
+                for (int r = tid / lw; r < rows; r += kPyrThreads / lw) {
+                    const unsigned d0 = px[r * pw + c], d1 = px[r * pw + c + 1];
+                    const unsigned e0 = d0 & 0x00ff00ffu, o0 = (d0 >> 8) & 0x00ff00ffu;
+                    const unsigned e1 = d1 & 0x00ff00ffu, o1 = (d1 >> 8) & 0x00ff00ffu;
+                    const unsigned em = (e0 >> 16) | (e1 << 16), om = (o0 >> 16) | (o1 << 16);
+                    hs[r * j.pairs + c] = e0 + e1 + 4u * (o0 + om) + 6u * em;
+                }
+        }
+        __syncthreads();
+        const bool more = i < n;
+        const int w = j.w[i], h1 = j.h[i - 1], y1 = yl[i - 1];
+        const int ox = more ? 2 * xl[i < kPyrLevels ? i + 1 : i] - 2 : xl[i];
+        const int halves = more ? (xh[i < kPyrLevels ? i + 1 : i] - xl[i < kPyrLevels ? i + 1 : i] + 1) / 2 * 2 + 2
+                                : pairs;
+        const int share = T << (n - i), sx = tx * share, sy = ty * share;
+        uint8_t* const dst = j.dst[i - 1];
+        const int lw = halves <= 16 ? 16 : halves <= 32 ? 32 : 64;
+        for (int y = yl[i] + tid / lw; y < yh[i]; y += kPyrThreads / lw) {
+            int r[5];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                r[k] = (reflect101(2 * y + k - 2, h1) - y1) * j.pairs;
+            }
+            for (int q = tid % lw; q < halves; q += lw) {
+                const int x = ox + 2 * q;
+                const auto column = [&](int c) {  // both sums of pair c
+                    return hs[r[0] + c] + hs[r[4] + c] + 4u * (hs[r[1] + c] + hs[r[3] + c]) +
+                           6u * hs[r[2] + c];
+                };
+                unsigned b;
+                if (x >= xl[i] && x + 1 < xh[i]) {
+                    b = pyr_round(column((x - xl[i]) >> 1), j.half_up);
+                    b = (b & 0xffu) | (b >> 8);
+                } else {
+                    b = 0;
+                    for (int k = 0; k < 2; ++k) {
+                        const int xr = min(max(reflect101(x + k, w), xl[i]), xh[i] - 1) - xl[i];
+                        const unsigned p = pyr_round(column(xr >> 1), j.half_up);
+                        b |= ((xr & 1) ? p >> 16 : p & 0xffu) << 8 * k;
+                    }
+                }
+                if (more) reinterpret_cast<uint16_t*>(px + (y - yl[i]) * pw)[q] = (uint16_t)b;
+                if (x >= sx && x < min(sx + share, w) && y >= sy && y < sy + share) {
+                    uint8_t* d = dst + (size_t)y * w + x;
+                    if (x + 1 < w) {
+                        const uint16_t both = (uint16_t)b;
+                        __builtin_memcpy(d, &both, 2);
+                    } else {
+                        *d = (uint8_t)b;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // ------------------------------------------------------------------ forward rows
@@ -1573,10 +1714,37 @@ hipError_t launch_init(unsigned* maxslots, int nslots, int* counter, hipStream_t
     return hipGetLastError();
 }
 
-hipError_t launch_pyr_down(const uint8_t* src, int sw, int sh, size_t spitch, uint8_t* dst,
-                           int dw, int dh, size_t dpitch, bool half_up, hipStream_t s) {
-    dim3 grid((dw + 127) / 128, dh);
-    k_pyr_down<<<grid, 128, 0, s>>>(src, sw, sh, spitch, dst, dw, dh, dpitch, half_up ? 1 : 0);
+hipError_t launch_pyr_down(const uint8_t* src, size_t spitch, uint8_t* const* dst, const int* w,
+                           const int* h, int n, bool half_up, hipStream_t s) {
+    if (n < 1 || n > kPyrLevels) return hipErrorInvalidValue;
+    if (n == 1) {
+        k_pyr_down<<<dim3((w[1] + 127) / 128, h[1]), 128, 0, s>>>(
+            src, w[0], h[0], spitch, dst[0], w[1], h[1], (size_t)w[1], half_up ? 1 : 0);
+        return hipGetLastError();
+    }
+    PyrJob j{};
+    j.src = src;
+    j.spitch = spitch;
+    for (int i = 0; i <= n; ++i) {
+        j.w[i] = w[i];
+        j.h[i] = h[i];
+        if (i) j.dst[i - 1] = dst[i - 1];
+    }
+    j.n = n;
+    j.half_up = half_up ? 1 : 0;
+    // 128 source pixels a side, halved while the chip would have fewer than one workgroup per
+    // CU: a small tile computes more of the levels below it twice (four levels: 1.8 times the
+    // source for 8 pixels, 3.2 for 4: 38 against 42 us at 3840 x 2160), but its chain of levels
+    // is shorter.
+    j.tile = 128 >> n;
+    const auto tiles = [&](int len) { return (len + j.tile - 1) / j.tile; };
+    while (j.tile > 4 && tiles(w[n]) * tiles(h[n]) < 256) j.tile /= 2;
+    int reach = j.tile;
+    for (int i = 1; i < n; ++i) reach = 2 * reach + 3;
+    j.pairs = (reach + 1) / 2;
+    j.rows = 2 * reach + 3;
+    k_pyr_levels<<<dim3(tiles(w[n]), tiles(h[n])), kPyrThreads,
+                   (size_t)j.rows * (2 * j.pairs + 1) * sizeof(unsigned), s>>>(j);
     return hipGetLastError();
 }
 

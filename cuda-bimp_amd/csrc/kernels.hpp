@@ -126,9 +126,12 @@ hipError_t prepare_size(int n);
 hipError_t prepare_common();
 
 hipError_t launch_init(unsigned* maxslots, int nslots, int* counter, hipStream_t s);
-// half_up: round (S + 128) >> 8 as OpenCV's host pyrDown; else half to even as its CUDA one
-hipError_t launch_pyr_down(const uint8_t* src, int sw, int sh, size_t spitch, uint8_t* dst,
-                           int dw, int dh, size_t dpitch, bool half_up, hipStream_t s);
+// Pyramid levels 1..n (n <= kPyrLevels) of a w[0] x h[0] frame, level i of w[i] = (w[i-1] + 1) / 2
+// columns, rows alike, at dst[i - 1], rows packed.  half_up: round (S + 128) >> 8 as OpenCV's
+// host pyrDown; else half to even as its CUDA one.
+constexpr int kPyrLevels = 4;
+hipError_t launch_pyr_down(const uint8_t* src, size_t spitch, uint8_t* const* dst, const int* w,
+                           const int* h, int n, bool half_up, hipStream_t s);
 hipError_t launch_fwd_rows(int FW, const uint8_t* img, size_t pitch, int H, int W,
                            const ScaleSet& ss, float scale, float2* R, int ldr, size_t rstride,
                            const float2* tw, hipStream_t s);
