@@ -286,10 +286,7 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
                          !(c->opt.flags & BIMP_FLAG_SINGLE_STREAM) &&
                          hipStreamIsCapturing(s, &capturing) == hipSuccess &&
                          capturing == hipStreamCaptureStatusNone;
-    if (useSide) {
-        HIPCHK(c, hipEventRecord(c->evFork, s));
-        HIPCHK(c, hipStreamWaitEvent(c->side, c->evFork, 0));
-    }
+    if (useSide) HIPCHK(c, hipEventRecord(c->evFork, s));
     const hipStream_t pq = useSide ? c->side : s;
     const uint8_t* lv[kMaxLevels] = {};
     size_t lp[kMaxLevels] = {};
@@ -299,16 +296,6 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
         lv[l] = c->level[l];
         lp[l] = (size_t)c->levelW[l];
     }
-    // the pyramid belongs to the upper-level part
-    for (int l = 0; l < c->maxLevel && part != kPartLevel0; l += bimpk::kPyrLevels) {
-        const int n = std::min(bimpk::kPyrLevels, c->maxLevel - l);
-        double bytes = (double)c->levelW[l] * c->levelH[l];
-        for (int k = 1; k <= n; ++k) bytes += (double)c->levelW[l + k] * c->levelH[l + k];
-        LaunchScope ls(c, pq, F_PYR, bytes);
-        HIPCHK(c, bimpk::launch_pyr_down(lv[l], lp[l], &c->level[l + 1], &c->levelW[l],
-                                         &c->levelH[l], n,
-                                         (c->opt.flags & BIMP_FLAG_RESIZE_CPU) != 0, pq));
-    }
     // the last step at pyramid level 0: the frame's final transforms on s
     const Step* lastL0 = nullptr;
     for (const Step& st : c->steps)
@@ -316,6 +303,49 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
             lastL0 = &st;
     auto on_side = [&](const Step& st) {
         return (st.direct ? c->sc[st.index].g.level : c->sc[c->groups[st.index].first].g.level) > 0;
+    };
+    // With a second stream, the forward passes of the frame's first level-0 group, which need
+    // the frame only, are issued before that stream's launches: they run while the host issues
+    // those, where the level-0 stream otherwise waited for it (1920 x 1080: 876 -> 842 us per
+    // frame, 3840 x 2160: 3554 -> 3490, 640 x 480: 250 -> 241).  Issuing all of level 0 first
+    // gave the same at 640 x 480, but its inverse passes fill the chip and leave a longer chain
+    // above them to the end (1237 x 701, five levels: 564 -> 581 us).
+    const Step* early = nullptr;
+    if (useSide && !c->steps.empty())
+        for (const Step& st : c->steps)
+            if (!early && !st.direct && !st.small && !on_side(st)) early = &st;
+    // The forward passes of an FFT step's group.
+    auto run_forward = [&](const Step& st) -> int {
+        const Group& gr = c->groups[st.index];
+        const auto& g = c->sc[gr.first].g;
+        // groups above level 0 own R2/T2 whenever the context has a side stream, on s as well
+        const bool upper = c->side && g.level > 0;
+        const hipStream_t q = upper && useSide ? c->side : s;
+        float2* const R = upper ? c->R2 : c->R;
+        const int ncols = g.FW / 2 + 1;
+        bimpk::ScaleSet ss;
+        ss.n = gr.n;
+        for (int k = 0; k < gr.n; ++k) {
+            const Scale& sk = c->sc[gr.first + k];
+            ss.kX[k] = sk.g.kX;
+            ss.G[k] = sk.G;
+            ss.DT[k] = sk.DT;
+            ss.C[k] = sk.C;
+        }
+        const size_t rstride = (size_t)g.H * ncols;
+        const double n = gr.n;
+        {
+            LaunchScope ls(c, q, F_FWD_ROWS, n * ((double)g.H * g.W + 8.0 * g.H * ncols), g.FW);
+            HIPCHK(c, bimpk::launch_fwd_rows(g.FW, lv[g.level], lp[g.level], g.H, g.W, ss,
+                                             c->opt.input_scale, R, ncols, rstride, c->tw[g.FW],
+                                             q));
+        }
+        {
+            LaunchScope ls(c, q, F_FWD_COLS, n * (8.0 * g.H * ncols + 8.0 * ncols * g.FH), g.FH);
+            HIPCHK(c, bimpk::launch_fwd_cols(g.FH, R, ncols, rstride, g.H, ss, ncols, c->tw[g.FH],
+                                             q));
+        }
+        return BIMP_OK;
     };
     auto run_step = [&](const Step& st) -> int {
         if (st.direct) {
@@ -355,31 +385,14 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
         // groups above level 0 own R2/T2 whenever the context has a side stream, on s as well
         const bool upper = c->side && g.level > 0;
         const hipStream_t q = upper && useSide ? c->side : s;
-        float2* const R = upper ? c->R2 : c->R;
         float2* const T = upper ? c->T2 : c->T;
         const size_t tCap = upper ? c->tCap2 : c->tCap;
         const int ncols = g.FW / 2 + 1;
         const float2* twW = c->tw[g.FW];
         const float2* twH = c->tw[g.FH];
-        bimpk::ScaleSet ss;
-        ss.n = gr.n;
-        for (int k = 0; k < gr.n; ++k) {
-            const Scale& sk = c->sc[gr.first + k];
-            ss.kX[k] = sk.g.kX;
-            ss.G[k] = sk.G;
-            ss.DT[k] = sk.DT;
-            ss.C[k] = sk.C;
-        }
-        const size_t rstride = (size_t)g.H * ncols;
-        const double n = gr.n;
-        {
-            LaunchScope ls(c, q, F_FWD_ROWS, n * ((double)g.H * g.W + 8.0 * g.H * ncols), g.FW);
-            HIPCHK(c, bimpk::launch_fwd_rows(g.FW, lv[g.level], lp[g.level], g.H, g.W, ss,
-                                             c->opt.input_scale, R, ncols, rstride, twW, q));
-        }
-        {
-            LaunchScope ls(c, q, F_FWD_COLS, n * (8.0 * g.H * ncols + 8.0 * ncols * g.FH), g.FH);
-            HIPCHK(c, bimpk::launch_fwd_cols(g.FH, R, ncols, rstride, g.H, ss, ncols, twH, q));
+        if (&st != early) {
+            const int r = run_forward(st);
+            if (r) return r;
         }
         // inverse passes over sub-batches of scales whose intermediate T fits the budget
         const Scale& s0 = c->sc[gr.first];
@@ -429,6 +442,21 @@ int run_filter(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, boo
         }
         return BIMP_OK;
     };
+    if (early) {
+        const int r = run_forward(*early);
+        if (r) return r;
+    }
+    if (useSide) HIPCHK(c, hipStreamWaitEvent(c->side, c->evFork, 0));
+    // the pyramid belongs to the upper-level part
+    for (int l = 0; l < c->maxLevel && part != kPartLevel0; l += bimpk::kPyrLevels) {
+        const int n = std::min(bimpk::kPyrLevels, c->maxLevel - l);
+        double bytes = (double)c->levelW[l] * c->levelH[l];
+        for (int k = 1; k <= n; ++k) bytes += (double)c->levelW[l + k] * c->levelH[l + k];
+        LaunchScope ls(c, pq, F_PYR, bytes);
+        HIPCHK(c, bimpk::launch_pyr_down(lv[l], lp[l], &c->level[l + 1], &c->levelW[l],
+                                         &c->levelH[l], n,
+                                         (c->opt.flags & BIMP_FLAG_RESIZE_CPU) != 0, pq));
+    }
     // Second-stream steps are issued first, so that the level-0 cells handed to that stream
     // below queue behind its own transforms rather than ahead of them.
     for (int pass = useSide ? 0 : 1; pass < 2; ++pass) {
