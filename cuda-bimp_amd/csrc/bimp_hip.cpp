@@ -123,6 +123,7 @@ void free_all(bimp_ctx* c) {
     (void)hipFree(c->blockMasks);
     (void)hipFree(c->nmsTable);
     (void)hipFree(c->kpBuf);
+    (void)hipHostFree(c->hostCount);  // and the records behind it
     if (c->hostIn) (void)hipHostFree(c->hostIn);
     if (c->hostInDone) (void)hipEventDestroy(c->hostInDone);
     for (auto& e : c->ev) {
@@ -162,6 +163,9 @@ constexpr int kDirectLaunchScales = 8;
 
 // Pyramid levels a context can hold (a frame side would have to exceed 2^31 to need more).
 constexpr int kMaxLevels = 32;
+// Keypoint records that come back with the count, in the call's one wait; later ones, with
+// larger frames, take a copy of their own.
+constexpr int kHostRecords = 8192;
 
 int inverse_batch(size_t tstride_elems) {
     const size_t per = tstride_elems * sizeof(float2);
@@ -516,8 +520,8 @@ int run_keypoints(bimp_ctx* c, void* out, int cap, int matrix_ld, hipStream_t s)
     {
         LaunchScope ls(c, s, F_NMS_WRITE, 4.0 * bimpk::kNmsThreads * c->totalBlocks);
         HIPCHK(c, bimpk::launch_nms_write(c->nmsTable, (int)c->sc.size(), c->totalBlocks,
-                                          c->blockCounts, c->counter, c->maxslots, c->blockMasks,
-                                          out, cap, matrix_ld, s));
+                                          c->blockCounts, c->counter, c->hostCount, c->maxslots,
+                                          c->blockMasks, out, cap, matrix_ld, s));
     }
     // the write pass cleared the slots: a later keypoint pass recomputes the maxima
     c->maxValid = false;
@@ -592,17 +596,23 @@ int keypoints_out(bimp_ctx* c, void* out, int cap, int matrix_ld, int out_on_dev
                                    matrix_ld, s)
                    : run_keypoints(c, target, cap, matrix_ld, s);
     if (st) return st;
-    int total = 0;
-    HIPCHK(c, hipMemcpyAsync(&total, c->counter, sizeof(int), hipMemcpyDeviceToHost, s));
+    const bool records = !out_on_device && cap > 0 && matrix_ld == 0;
+    const int early = records ? std::min(cap, kHostRecords) : 0;
+    if (early)
+        HIPCHK(c, bimpk::launch_records_out(c->counter, early, target, sizeof(bimp_keypoint) / 4,
+                                            c->hostRecords, s));
     HIPCHK(c, hipStreamSynchronize(s));
+    const int total = *static_cast<volatile int*>(c->hostCount);
     const int n = std::min(total, cap);
-    if (!out_on_device && n > 0) {
-        if (matrix_ld > 0) {
-            HIPCHK(c, hipMemcpy2D(out, (size_t)matrix_ld * 4, target, (size_t)matrix_ld * 4,
-                                  (size_t)n * 4, BIMP_KP_VECTOR_LENGTH, hipMemcpyDeviceToHost));
-        } else {
-            HIPCHK(c, hipMemcpy(out, target, (size_t)n * elem, hipMemcpyDeviceToHost));
-        }
+    if (records && n > 0) {
+        const int m = std::min(n, early);
+        std::memcpy(out, c->hostRecords, (size_t)m * elem);
+        if (n > m)
+            HIPCHK(c, hipMemcpy((bimp_keypoint*)out + m, (bimp_keypoint*)target + m,
+                                (size_t)(n - m) * elem, hipMemcpyDeviceToHost));
+    } else if (!out_on_device && n > 0) {
+        HIPCHK(c, hipMemcpy2D(out, (size_t)matrix_ld * 4, target, (size_t)matrix_ld * 4,
+                              (size_t)n * 4, BIMP_KP_VECTOR_LENGTH, hipMemcpyDeviceToHost));
     }
     if (count) *count = total;
     if (c->opt.flags & BIMP_FLAG_PROFILE) collect_profile(c);
@@ -1099,6 +1109,16 @@ int bimp_create(int width, int height, const float* lambdas, int n, const bimp_o
         dalloc(&c->blockMasks, (size_t)blocks * bimpk::kNmsThreads) != hipSuccess ||
         dalloc(&c->maxslots, c->sc.size()) != hipSuccess || dalloc(&c->counter, 1) != hipSuccess)
         return bail(BIMP_E_ALLOC, "nms buffers");
+    {
+        const size_t head = 256;
+        char* p = nullptr;
+        if (hipHostMalloc((void**)&p, head + kHostRecords * sizeof(bimp_keypoint),
+                          hipHostMallocDefault) != hipSuccess)
+            return bail(BIMP_E_ALLOC, "pinned keypoint records");
+        c->hostCount = (int*)p;
+        *c->hostCount = 0;
+        c->hostRecords = (bimp_keypoint*)(p + head);
+    }
     if (hipMemset(c->maxslots, 0, c->sc.size() * sizeof(unsigned)) != hipSuccess ||
         hipMemset(c->counter, 0, sizeof(int)) != hipSuccess)
         return bail(BIMP_E_DEVICE, "nms buffers");

@@ -94,6 +94,10 @@ struct bimp_ctx {
     // event after its last upload, waited on before the staging is rewritten
     uint8_t* hostIn = nullptr;
     hipEvent_t hostInDone = nullptr;
+    // pinned memory that the device writes: the frame's keypoint count and, behind it, the first
+    // kHostRecords records
+    int* hostCount = nullptr;
+    bimp_keypoint* hostRecords = nullptr;
     bool maxValid = false;
     // the per-scale max slots are zero at this point of the stream (set at creation and by
     // the keypoint pass, which clears them once it has read them): a frame then needs no reset

@@ -172,10 +172,14 @@ hipError_t launch_nms_count(const NmsScale* scales, int nscales, int total_block
                             const unsigned* maxslots, double thresh, int* block_counts,
                             unsigned* masks, hipStream_t s);
 hipError_t launch_nms_write(const NmsScale* scales, int nscales, int total_blocks,
-                            const int* block_counts, int* counter, unsigned* maxslots,
+                            const int* block_counts, int* counter, int* host_count,
+                            unsigned* maxslots,
                             const unsigned* masks, void* out, int cap, int matrix_ld,
                             hipStream_t s);
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
+// min(*count, cap) records of `words` 4-byte words into pinned host memory.
+hipError_t launch_records_out(const int* count, int cap, const void* records, int words,
+                              void* host, hipStream_t s);
 hipError_t launch_bgr_to_gray(const uint8_t* bgr, size_t bpitch, int w, int h, uint8_t* gray,
                               size_t gpitch, hipStream_t s);
 // dst[0] = counter[0] on the stream (a kernel, so that it can sit in a captured graph).
