@@ -211,15 +211,18 @@ struct RowCfg {
 // both are separated with Z(k) and conj(Z(N-k)).  Columns beyond W repeat column W-1 for kX
 // samples, then column 0 (padDataClampToBorder, convolutionFFT2D.cuh:56-85).  blockIdx.y
 // selects the scale of the batch (scales of one pyramid level differ only in kX).  Pixels are
-// uint8 (detection) or float (the differentiation form's images); pitch counts pixels.
+// uint8 (detection) or float (the differentiation form's images, `per` scales of each, istride
+// apart); pitch counts pixels.
 template <int FW, class Pix>
-__global__ void __launch_bounds__(RowCfg<FW>::THREADS) k_fwd_rows(const Pix* __restrict__ img, size_t pitch,
+__global__ void __launch_bounds__(RowCfg<FW>::THREADS) k_fwd_rows(const Pix* __restrict__ img, size_t istride,
+                                                 int per, size_t pitch,
                                                  int H, int W, ScaleSet ss, float scale,
                                                  float2* __restrict__ Rbase, int ldr,
                                                  size_t rstride, const float2* __restrict__ tw) {
     using C = FFTCfg<FW>;
     extern __shared__ float lds[];
     const int sidx = blockIdx.y;
+    if constexpr (std::is_same<Pix, float>::value) img += (size_t)(sidx / per) * istride;
     const int kX = ss.kX[sidx];
     float2* R = Rbase + (size_t)sidx * rstride;
     const int g = threadIdx.x / C::TPV, lane = threadIdx.x % C::TPV;
@@ -1766,16 +1769,16 @@ hipError_t launch_pyr_down(const uint8_t* src, size_t spitch, uint8_t* const* ds
 }
 
 template <class Pix>
-static hipError_t fwd_rows(int FW, const Pix* img, size_t pitch, int H, int W, const ScaleSet& ss,
-                           float scale, float2* R, int ldr, size_t rstride, const float2* tw,
-                           hipStream_t s) {
+static hipError_t fwd_rows(int FW, const Pix* img, size_t istride, int per, size_t pitch, int H,
+                           int W, const ScaleSet& ss, float scale, float2* R, int ldr,
+                           size_t rstride, const float2* tw, hipStream_t s) {
 #define X(N)                                                                                 \
     if (FW == N) {                                                                           \
         const int vpb = RowCfg<N>::VPB;                                                      \
         const int pairs = (H + 1) / 2;                                                       \
         dim3 grid((pairs + vpb - 1) / vpb, ss.n);                                            \
         k_fwd_rows<N, Pix><<<grid, RowCfg<N>::THREADS, vpb * N * sizeof(float2), s>>>(       \
-            img, pitch, H, W, ss, scale, R, ldr, rstride, tw);                               \
+            img, istride, per, pitch, H, W, ss, scale, R, ldr, rstride, tw);                 \
         return hipGetLastError();                                                            \
     }
     BIMP_FOR_SIZES(X)
@@ -1786,13 +1789,13 @@ static hipError_t fwd_rows(int FW, const Pix* img, size_t pitch, int H, int W, c
 hipError_t launch_fwd_rows(int FW, const uint8_t* img, size_t pitch, int H, int W,
                            const ScaleSet& ss, float scale, float2* R, int ldr, size_t rstride,
                            const float2* tw, hipStream_t s) {
-    return fwd_rows(FW, img, pitch, H, W, ss, scale, R, ldr, rstride, tw, s);
+    return fwd_rows(FW, img, 0, ss.n, pitch, H, W, ss, scale, R, ldr, rstride, tw, s);
 }
 
-hipError_t launch_fwd_rows_f32(int FW, const float* img, size_t pitch, int H, int W,
-                               const ScaleSet& ss, float scale, float2* R, int ldr,
+hipError_t launch_fwd_rows_f32(int FW, const float* img, size_t istride, int per, size_t pitch,
+                               int H, int W, const ScaleSet& ss, float scale, float2* R, int ldr,
                                size_t rstride, const float2* tw, hipStream_t s) {
-    return fwd_rows(FW, img, pitch, H, W, ss, scale, R, ldr, rstride, tw, s);
+    return fwd_rows(FW, img, istride, per, pitch, H, W, ss, scale, R, ldr, rstride, tw, s);
 }
 
 hipError_t launch_fwd_cols(int FH, const float2* R, int ldr, size_t rstride, int H,

@@ -11,15 +11,19 @@ constexpr int kNumOri = 8;
 constexpr int kUniqueOri = 5;  // orientations 5..7 mirror 3..1 in the spectrum
 
 // Scales of one resolution group (same pyramid level and transform size) processed by one
-// launch of each FFT stage.
+// launch of each FFT stage: at most kMaxBatch, and in the differentiation form those of several
+// images, kMaxEntries (scale, image) pairs in all.
 constexpr int kMaxBatch = 8;
-struct ScaleSet {
+constexpr int kMaxEntries = 32;
+template <int M>
+struct ScaleSetOf {
     int n;
-    int kX[kMaxBatch];       // kernel centre = clamp-padding width
-    const float* G[kMaxBatch];
-    float2* DT[kMaxBatch];
-    float* C[kMaxBatch];
+    int kX[M];  // kernel centre = clamp-padding width
+    const float* G[M];
+    float2* DT[M];
+    float* C[M];
 };
+using ScaleSet = ScaleSetOf<kMaxEntries>;
 
 // A resolution group whose stages run in one launch each with those of other groups (all
 // transforms of at most 512 points).
@@ -35,7 +39,7 @@ struct SmallJob {
     float2 *R, *T;      // the group's own intermediates
     size_t rstride, tstride;
     const float2 *twW, *twH;
-    ScaleSet ss;
+    ScaleSetOf<kMaxBatch> ss;
 };
 struct SmallJobs {
     SmallJob j[kSmallJobs];
@@ -135,9 +139,10 @@ hipError_t launch_pyr_down(const uint8_t* src, size_t spitch, uint8_t* const* ds
 hipError_t launch_fwd_rows(int FW, const uint8_t* img, size_t pitch, int H, int W,
                            const ScaleSet& ss, float scale, float2* R, int ldr, size_t rstride,
                            const float2* tw, hipStream_t s);
-// The same pass over a float image (pitch in floats), e.g. a differentiation-form level.
-hipError_t launch_fwd_rows_f32(int FW, const float* img, size_t pitch, int H, int W,
-                               const ScaleSet& ss, float scale, float2* R, int ldr,
+// The same pass over float images (pitch in floats), e.g. a differentiation-form level: entry k
+// of ss is of image k / per, `istride` floats apart.
+hipError_t launch_fwd_rows_f32(int FW, const float* img, size_t istride, int per, size_t pitch,
+                               int H, int W, const ScaleSet& ss, float scale, float2* R, int ldr,
                                size_t rstride, const float2* tw, hipStream_t s);
 hipError_t launch_fwd_cols(int FH, const float2* R, int ldr, size_t rstride, int H,
                            const ScaleSet& ss, int ncols, const float2* tw, hipStream_t s);
