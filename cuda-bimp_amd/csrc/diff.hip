@@ -468,7 +468,51 @@ __device__ __forceinline__ bool valid(int x, int y, int a, int b, int W, int H) 
 //   bit o: ds > 0, bit 8 + o: tangential > 0, bit 16 + o: v2 > 0 and v1 > 0, bit 24 + o: v2 > 0
 // stored with g as one 8-byte pair per pixel of H x FW (zero right of the data).  Four
 // float masks per pixel and orientation took 16 times the bytes: 92 us to write and 96 us to
-// gather from per scale of eight 512 x 512 images, against 55 us here.  blockIdx.z: entry.
+// gather from per scale of eight 512 x 512 images, against 55 us here.
+// EDGE: pixels near the frame's edge test each orientation's reach and wrap their reads; a
+// wavefront whose 64 pixels lie inside every reach does neither.  Bound by instructions: 32
+// entries of 512 x 512 and 32 of 256 x 256 took 254 us with the tests everywhere, 212 so.
+template <bool EDGE>
+__device__ __forceinline__ unsigned branch_bits(const float* __restrict__ C, size_t mp, int P,
+                                                int FW, int H, int W, const CellParams& p, int x,
+                                                int y) {
+    const int g0 = y * FW + x;
+    auto cat = [&](const float* m, int idx) {
+        if (EDGE) {
+            if (idx >= P) idx -= P;
+            if (idx < 0) idx += P;
+        }
+        return m[(unsigned)idx];
+    };
+    unsigned bits = 0;
+#pragma unroll
+    for (int o = 0; o < kNumOri; ++o) {
+        const float* Co = C + o * mp;
+        const float* C2 = C + ((o + kNumOri / 2) % kNumOri) * mp;
+        const float c = Co[(unsigned)g0];
+        const int a = p.ea[o], b = p.eb[o];
+        if (!EDGE || valid(x, y, a, b, W, H)) {
+            const int d1 = 2 * b - 2 * a * FW;
+            const float v = (float)((double)c - 0.5 * (double)cat(Co, g0 + d1) -
+                                    0.5 * (double)cat(Co, g0 - d1));
+            if (v > 0.f) bits |= 1u << o;
+        }
+        const int ia = p.ia[o], ib = p.ib[o];
+        if (!EDGE || valid(x, y, ia, ib, W, H)) {
+            const float vt = cat(Co, g0 - ia * FW - ib) - c;
+            if (vt > 0.f) bits |= 1u << (8 + o);
+            const int rr = p.ra[o] * FW + p.rb[o];
+            float v1 = c - 16.f * cat(C2, g0 + rr);
+            const bool m1 = v1 > 0.f;
+            v1 = m1 ? v1 : 0.f;
+            const float v2 = v1 + c - 16.f * cat(C2, g0 - rr);
+            if (v2 > 0.f) bits |= (1u << (24 + o)) | (m1 ? 1u << (16 + o) : 0u);
+        }
+    }
+    return bits;
+}
+
+// blockIdx.z: entry.
 __global__ void __launch_bounds__(256) k_branch_bits(const float* __restrict__ C, int Hc, int FH,
                                                      int FW, int H, int W, AdjSet set,
                                                      const float* __restrict__ gD, size_t gstride,
@@ -480,44 +524,28 @@ __global__ void __launch_bounds__(256) k_branch_bits(const float* __restrict__ C
     // complex-cell maps are read with the reference's linear index y*FW + x over the FH x FW
     // array, wrapping past the end (the forward stencil's semantics); they hold Hc rows, which
     // is all that valid pixels reach
-    const int P = FH * FW, g0 = y * FW + x;
+    const int P = FH * FW;
     const size_t mp = (size_t)Hc * FW;
     C += (size_t)entry * kNumOri * mp;
     gD += (size_t)(entry / set.n) * gstride + set.resp[j];
-    auto cat = [&](const float* m, int idx) {
-        if (idx >= P) idx -= P;
-        if (idx < 0) idx += P;
-        return m[(unsigned)idx];
-    };
+    int ra = 0, rb = 0;  // the widest reach (the r taps lie inside the i taps')
+#pragma unroll
+    for (int o = 0; o < kNumOri; ++o) {
+        ra = max(ra, max(abs(p.ea[o]), abs(p.ia[o])));
+        rb = max(rb, max(abs(p.eb[o]), abs(p.ib[o])));
+    }
+    const int xw = __builtin_amdgcn_readfirstlane(x);  // the wavefront's first pixel
+    // reads stay in rows 0..H-1 and columns 0..W-1 (a valid pixel may reach row H or column W,
+    // one past the data, which wraps where the data fills the padded array)
+    const bool inside =
+            valid(xw, y, ra, rb, W - 1, H - 1) && valid(xw + 63, y, ra, rb, W - 1, H - 1);
     const float g = x < W ? gD[(size_t)y * W + x] : 0.f;
     unsigned bits = 0;
-    if (g != 0.f) {
-#pragma unroll
-        for (int o = 0; o < kNumOri; ++o) {
-            const float* Co = C + o * mp;
-            const float* C2 = C + ((o + kNumOri / 2) % kNumOri) * mp;
-            const float c = Co[(unsigned)g0];
-            const int a = p.ea[o], b = p.eb[o];
-            if (valid(x, y, a, b, W, H)) {
-                const int d1 = 2 * b - 2 * a * FW;
-                const float v = (float)((double)c - 0.5 * (double)cat(Co, g0 + d1) -
-                                        0.5 * (double)cat(Co, g0 - d1));
-                if (v > 0.f) bits |= 1u << o;
-            }
-            const int ia = p.ia[o], ib = p.ib[o];
-            if (valid(x, y, ia, ib, W, H)) {
-                const float vt = cat(Co, g0 - ia * FW - ib) - c;
-                if (vt > 0.f) bits |= 1u << (8 + o);
-                const int rr = p.ra[o] * FW + p.rb[o];
-                float v1 = c - 16.f * cat(C2, g0 + rr);
-                const bool m1 = v1 > 0.f;
-                v1 = m1 ? v1 : 0.f;
-                const float v2 = v1 + c - 16.f * cat(C2, g0 - rr);
-                if (v2 > 0.f) bits |= (1u << (24 + o)) | (m1 ? 1u << (16 + o) : 0u);
-            }
-        }
-    }
-    out[(size_t)entry * H * FW + g0] = make_uint2(__float_as_uint(g), bits);
+    if (inside)
+        bits = branch_bits<false>(C, mp, P, FW, H, W, p, x, y);
+    else if (g != 0.f)
+        bits = branch_bits<true>(C, mp, P, FW, H, W, p, x, y);
+    out[(size_t)entry * H * FW + y * FW + x] = make_uint2(__float_as_uint(g), g != 0.f ? bits : 0u);
 }
 
 // Pass 2, in the load of gZ's row transforms: gathers, for a map position q and orientation o,

@@ -37,3 +37,35 @@ def test_batch_equals_single_images(B, w, h, bank, n):
                           for i in range(n)])
     assert np.all(np.isfinite(one))
     assert np.array_equal(got.view(np.uint32), one.view(np.uint32))
+
+
+def _backward(B, d, imgs, up):
+    x, g, out = (B.DeviceBuffer(a.nbytes) for a in (imgs, up, imgs))
+    x.upload(imgs)
+    g.upload(up)
+    gp = d.backward(x.ptr.value, len(imgs), g.ptr.value, out.ptr.value)
+    return out.download(np.zeros_like(imgs)), gp
+
+
+# frames that fill the padded array or not, with wavefronts inside every tap's reach and without,
+# in launches that fill all 32 pairs; the reference gradient of one image pins the branch bits
+@pytest.mark.parametrize("w,h,n", [(256, 256, 8), (512, 128, 8), (300, 256, 3), (320, 200, 2)])
+def test_backward_inside_and_at_the_edges(B, w, h, n):
+    from diff_ref import DiffRef
+    lam = O.BASE_BANK[:4]
+    imgs = np.stack([O.synth_frame(w, h, 15, 40 + i) for i in range(n)]).astype(np.float32)
+    imgs /= np.float32(255)
+    d = B.Diff(w, h, lam)
+    up = np.random.default_rng(2).standard_normal((n, d.response_size)).astype(np.float32)
+    ref = DiffRef(w, h, lam)
+    targets = ref.forward(imgs[-1].astype(np.float64), gamma=0.6)
+    _, rg, rp = ref.gradient(imgs[-1].astype(np.float64), targets)
+    up[-1] = np.concatenate([2 * (a - b).ravel() for a, b in
+                             zip(ref.forward(imgs[-1].astype(np.float64)), targets)])
+    gi, _ = _backward(B, d, imgs, up)
+    for i in range(n):
+        one, gp = _backward(B, d, imgs[i:i + 1], up[i:i + 1])
+        assert np.array_equal(gi[i].view(np.uint32), one[0].view(np.uint32)), i
+    # the bars of the form's own gradient tests
+    assert np.linalg.norm(one[0] - rg) <= 1e-3 * np.linalg.norm(rg)
+    assert np.all(np.abs(gp - rp) <= 1e-3 * np.abs(rp))
