@@ -253,6 +253,48 @@ __global__ void __launch_bounds__(RowCfg<FW>::THREADS) k_fwd_rows(const Pix* __r
     }
 }
 
+// ------------------------------------------------------------------ buffer access
+// Raw buffer loads and stores: one 32-bit lane offset and a scalar or constant part per access
+// where pointers take a 64-bit vector addition each, and a store beyond the buffer's size is
+// dropped by the hardware, so a row's end costs no compare and no branch.  The range check
+// compares lane offset plus constant with the size, so stores that rely on it pass no scalar
+// offset.
+// In k_inv_cols this takes 1536 points from 1241 to 1093 vector instructions and from 96 to 90
+// registers: 274 -> 266 us per 1920 x 1080 frame, 1024 points 105 -> 100 us per 1024 x 1024 frame
+// and 2560 points 1041 -> 1030 us per 3840 x 2160 frame.  The row kernels keep pointers and
+// compares: on buffers k_inv_rows<2048> took 204 us instead of 195 and <4096> 1183 instead of
+// 1058, every square root and store then waiting for the last butterfly.
+using BufferRsrc = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ BufferRsrc buffer_of(const void* p, unsigned bytes) {
+    constexpr int kRaw32 = 0x00027000;  // untyped 32-bit data
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, kRaw32);
+}
+constexpr unsigned kWholeBuffer = 0x7fffffffu;
+constexpr unsigned kDropStore = 0x80000000u;  // a lane offset beyond any buffer here
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float2 buffer_load_f2(BufferRsrc r, unsigned lane_bytes, int bytes) {
+    const uint2v x = __builtin_amdgcn_raw_buffer_load_b64(r, (int)lane_bytes, bytes, 0);
+    return make_float2(__uint_as_float(x.x), __uint_as_float(x.y));
+}
+__device__ __forceinline__ float buffer_load_f1(BufferRsrc r, unsigned lane_bytes, int bytes) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)lane_bytes, bytes, 0));
+}
+__device__ __forceinline__ void buffer_store_f2(BufferRsrc r, unsigned lane_bytes, float2 v) {
+    const uint2v x = {__float_as_uint(v.x), __float_as_uint(v.y)};
+    __builtin_amdgcn_raw_buffer_store_b64(x, r, (int)lane_bytes, 0, 0);
+}
+// a * s rounded once, never contracted into the transform's first additions: the results do not
+// depend on how the loads before it are arranged.
+__device__ __forceinline__ float2 scale1(float2 a, float s) {
+#pragma clang fp contract(off)
+    return make_float2(a.x * s, a.y * s);
+}
+// Constant byte offset c as a page in the scalar operand and the rest in the instruction.
+template <class F>
+__device__ __forceinline__ auto paged(unsigned lane_bytes, int c, F f) {
+    return f(lane_bytes + (unsigned)(c & 4095), c & ~4095);
+}
+
 // ------------------------------------------------------------------ column kernels
 // A workgroup owns CB adjacent columns; global row-major data moves through LDS (stride
 // N + 8 float2 per column keeps the transposing accesses conflict-free) so that every global
@@ -431,28 +473,34 @@ __global__ void __launch_bounds__(ColCfg<FH>::THREADS) k_inv_cols(
         // direct: column kx = k0 + g; partner: stored column kx = k0 + 1 + g, output FW - kx
         const int kx = k0 + partner + g;
         const bool ok = partner ? (kx < half) : (kx <= half);
-        const float2* dcol = DT + (size_t)(ok ? kx : 0) * FH;
         // bank column: direct o <= 4 -> kx, o >= 5 -> FW-kx; partner o <= 4 -> FW-kx, else kx
         const int cg = ((o <= 4) != (partner != 0)) ? kx : (kx == 0 ? 0 : FW - kx);
-        const float* gcol = G + ((size_t)og * FW + (ok ? cg : 0)) * FH;
-        // D * G_o: per-lane base pointers, element offsets in_index(e, 0) known at compile
-        // time; the partner pass reads G at row FH - ky, except ky = 0 (lane 0 of e = 0)
+        // D * G_o: rows in_index(e, lane) of one stored column and one bank column, constant
+        // offsets from one lane offset each; the partner pass reads G at row FH - ky, except
+        // ky = 0 (lane 0 of e = 0)
+        const BufferRsrc rd = buffer_of(DT, kWholeBuffer);
+        const BufferRsrc rg = buffer_of(G + (size_t)og * FW * FH, kWholeBuffer);
+        const unsigned od = (unsigned)((ok ? kx : 0) * FH + lane) * 8u;
+        const unsigned cgo = (unsigned)((ok ? cg : 0) * FH);
+        const auto ld2 = [&](unsigned lo, int so) { return buffer_load_f2(rd, lo, so); };
+        const auto ld1 = [&](unsigned lo, int so) { return buffer_load_f1(rg, lo, so); };
         float2 v[C::E];
-        const float2* dl = dcol + lane;
         if (partner) {
-            const float* gl = gcol + (FH - lane);
+            const unsigned o0 = (cgo + (lane ? FH - lane : 0)) * 4u;
+            const unsigned ol = (cgo + (C::TPV - 1 - lane)) * 4u;
 #pragma unroll
             for (int e = 0; e < C::E; ++e) {
                 const int ce = in_index<FH>(e, 0);
-                const float gv = e == 0 ? gcol[lane ? FH - lane : 0] : gl[-ce];
-                v[e] = cscale(dl[ce], gv);
+                const float gv = e == 0 ? buffer_load_f1(rg, o0, 0)
+                                        : paged(ol, (FH - (C::TPV - 1) - ce) * 4, ld1);
+                v[e] = scale1(paged(od, ce * 8, ld2), gv);
             }
         } else {
-            const float* gl = gcol + lane;
+            const unsigned ol = (cgo + lane) * 4u;
 #pragma unroll
             for (int e = 0; e < C::E; ++e) {
                 const int ce = in_index<FH>(e, 0);
-                v[e] = cscale(dl[ce], gl[ce]);
+                v[e] = scale1(paged(od, ce * 8, ld2), paged(ol, ce * 4, ld1));
             }
         }
         if constexpr (IC::LDS_TW)
@@ -468,12 +516,12 @@ __global__ void __launch_bounds__(ColCfg<FH>::THREADS) k_inv_cols(
         const int slot = partner ? CB - 1 - g : g;
         const int base = partner ? FW - k0 - CB : k0;
         // a thread stores column b of the block, rows yy0 + i*YS (IC::THREADS is a multiple
-        // of CB); where a round takes 8 or more such rows, four LDS reads go out before their
-        // four stores instead of one read waiting before each store
+        // of CB), up to four LDS reads going out before their stores instead of one read
+        // waiting before each store
         static_assert(IC::THREADS % CB == 0, "whole rows of the block per pass");
         constexpr int YS = IC::THREADS / CB, IT = (IC::BRG + YS - 1) / YS;
         constexpr int J = IT % 4 == 0 ? 4 : IT % 3 == 0 ? 3 : IT % 2 == 0 ? 2 : 1;
-        constexpr bool BATCH = IT >= 6 && J > 1 && IC::BRG % YS == 0;
+        constexpr bool BATCH = IC::BRG % YS == 0;
         const int b = threadIdx.x % CB, yy0 = threadIdx.x / CB;
         const int ks = partner ? k0 + CB - b : k0 + b;  // stored column
         const bool wcol = partner ? (ks < half) : (ks <= half);
@@ -492,24 +540,25 @@ __global__ void __launch_bounds__(ColCfg<FH>::THREADS) k_inv_cols(
             __syncthreads();
             // T is column-block-major: block base / CB holds rows 0..Hc-1 of its CB columns
             // contiguously, so a unit's rows go out as one contiguous run
-            float2* const blk = To + (size_t)(base / CB) * Hc * CB;
+            float2* const blk = To + ((size_t)(base / CB) * Hc + ylo) * CB;
             if constexpr (BATCH) {
+                const BufferRsrc rt = buffer_of(blk, (unsigned)rows * (CB * 8u));
+                const unsigned ot = wcol ? (unsigned)threadIdx.x * 8u : kDropStore;
 #pragma unroll 1
                 for (int i0 = 0; i0 < IT; i0 += J) {
                     float2 val[J];
 #pragma unroll
                     for (int j = 0; j < J; ++j) val[j] = lds2[b * IC::SS + yy0 + (i0 + j) * YS];
-                    float2* dst = blk + (size_t)(ylo + yy0 + i0 * YS) * CB + b;
 #pragma unroll
                     for (int j = 0; j < J; ++j)
-                        if (wcol && yy0 + (i0 + j) * YS < rows) dst[(size_t)j * YS * CB] = val[j];
+                        buffer_store_f2(rt, ot + (unsigned)(i0 + j) * (YS * CB * 8u), val[j]);
                 }
             } else {
                 for (int t = threadIdx.x; t < rows * CB; t += IC::THREADS) {
                     const int bt = t % CB, yy = t / CB;
                     const int kst = partner ? k0 + CB - bt : k0 + bt;  // stored column
                     const bool w = partner ? (kst < half) : (kst <= half);
-                    if (w) blk[(size_t)(ylo + yy) * CB + bt] = lds2[bt * IC::SS + yy];
+                    if (w) blk[(size_t)yy * CB + bt] = lds2[bt * IC::SS + yy];
                 }
             }
         }
