@@ -495,7 +495,8 @@ int run_cells(bimp_ctx* c, hipStream_t s) {
     return BIMP_OK;
 }
 
-int run_keypoints(bimp_ctx* c, void* out, int cap, int matrix_ld, hipStream_t s) {
+// host_count: pinned memory for the total as well, or null where the caller reads it on the device
+int run_keypoints(bimp_ctx* c, void* out, int cap, int matrix_ld, int* host_count, hipStream_t s) {
     if (!c->maxValid) {
         {
             LaunchScope ls(c, s, F_INIT, 0);
@@ -520,7 +521,7 @@ int run_keypoints(bimp_ctx* c, void* out, int cap, int matrix_ld, hipStream_t s)
     {
         LaunchScope ls(c, s, F_NMS_WRITE, 4.0 * bimpk::kNmsThreads * c->totalBlocks);
         HIPCHK(c, bimpk::launch_nms_write(c->nmsTable, (int)c->sc.size(), c->totalBlocks,
-                                          c->blockCounts, c->counter, c->hostCount, c->maxslots,
+                                          c->blockCounts, c->counter, host_count, c->maxslots,
                                           c->blockMasks, out, cap, matrix_ld, s));
     }
     // the write pass cleared the slots: a later keypoint pass recomputes the maxima
@@ -594,7 +595,7 @@ int keypoints_out(bimp_ctx* c, void* out, int cap, int matrix_ld, int out_on_dev
     }
     int st = frame ? run_frame_any(c, frame->img, frame->pitch, frame->on_device, target, cap,
                                    matrix_ld, s)
-                   : run_keypoints(c, target, cap, matrix_ld, s);
+                   : run_keypoints(c, target, cap, matrix_ld, c->hostCount, s);
     if (st) return st;
     const bool records = !out_on_device && cap > 0 && matrix_ld == 0;
     const int early = records ? std::min(cap, kHostRecords) : 0;
@@ -665,7 +666,7 @@ int build_frame_graph(bimp_ctx* c, const uint8_t* src, size_t pitch, void* out, 
     };
     auto kp = [](bimp_ctx* x, hipStream_t q, void* a) {
         const GraphArgs* g = static_cast<const GraphArgs*>(a);
-        return run_keypoints(x, g->out, g->cap, g->ld, q);
+        return run_keypoints(x, g->out, g->cap, g->ld, x->hostCount, q);
     };
     const bool split = c->side && !(c->opt.flags & BIMP_FLAG_SINGLE_STREAM);
     hipGraph_t parts[4] = {nullptr, nullptr, nullptr, nullptr};  // head, upper, level 0, tail
@@ -720,7 +721,7 @@ int run_frame_any(bimp_ctx* c, const uint8_t* img, size_t pitch, int on_device, 
                   int cap, int ld, hipStream_t s) {
     if (!(c->opt.flags & BIMP_FLAG_GRAPH) || (c->opt.flags & BIMP_FLAG_PROFILE)) {
         int st = run_filter(c, img, pitch, on_device, true, s);
-        return st ? st : run_keypoints(c, out, cap, ld, s);
+        return st ? st : run_keypoints(c, out, cap, ld, c->hostCount, s);
     }
     const uint8_t* src = img;
     size_t p = pitch;
@@ -786,7 +787,7 @@ int bimpi::run_frame(bimp_ctx* c, const uint8_t* d_img, size_t pitch, void* out,
                      int matrix_ld, hipStream_t s) {
     const int st = run_filter(c, d_img, pitch, 1, true, s);
     if (st) return st;
-    return run_keypoints(c, out, cap, matrix_ld, s);
+    return run_keypoints(c, out, cap, matrix_ld, nullptr, s);
 }
 
 // ======================================================================= C ABI

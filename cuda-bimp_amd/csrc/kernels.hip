@@ -1472,7 +1472,7 @@ __global__ void __launch_bounds__(kNmsThreads) k_nms_write(
     if (last) {
         if (threadIdx.x == 0) {
             *counter = start + mine;
-            *host_count = start + mine;
+            if (host_count) *host_count = start + mine;
         }
         for (int i = (int)threadIdx.x; i < nscales; i += kNmsThreads) maxslots[i] = 0u;
     }
