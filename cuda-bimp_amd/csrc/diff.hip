@@ -380,7 +380,8 @@ __global__ void __launch_bounds__(kRowThreads) k_pad_rows(const float* __restric
 // layout of T.  Workgroups are dealt round-robin to the eight XCDs; the numbering gives each
 // XCD every eighth column block, its eight orientations back to back (D's columns from L2 after
 // the first), then the images of one scale (that XCD's share of Q stays in its L2), then the
-// scales: 208 us for 32 entries of 512 x 512, 224 us with each orientation on one XCD.
+// scales: 194 us for 32 entries of 512 x 512 (208 when first measured, against 224 with each
+// orientation on one XCD).
 template <int N>
 __global__ void __launch_bounds__(ACfg<N>::THREADS) k_z_cols(const float2* __restrict__ D,
                                                              AdjSet set, int nb, int W, int Hc,
@@ -554,7 +555,7 @@ __global__ void __launch_bounds__(256) k_branch_bits(const float* __restrict__ C
 //   R_o(x) = relu(relu(C_o(x) - 16 C_o'(x+r)) + C_o(x) - 16 C_o'(x-r)), o' = o+4,
 // then gZ = gC * Z / |Z| (zero where |Z| = 0) and the forward row transform into T's layout.
 // Bound by HBM (Z in, T out: 212 us at the copy rate for four scales of eight 512 x 512 images);
-// takes 409 us, of which the gather is 165.
+// takes 392 us, of which the gather is about 160.
 struct Gather {
     const uint2* gm;  // (g, branch bits), H rows of FW
     int P, HF;        // FH*FW, H*FW
