@@ -66,6 +66,11 @@ struct bimp_diff {
     float* partials = nullptr;
     int maxBlocks = 0;
     int nbMax = 8;  // images whose pyramids are held at once
+    // the end of the last forward on a stream other than the null stream, recorded there: a
+    // parameter change waits for it
+    hipEvent_t fwdDone = nullptr;
+    bool fwdPending = false;   // fwdDone marks a forward that nothing has waited for
+    bool fwdCaptured = false;  // a forward sits in a caller's graph, whose replays mark nothing
     std::string err;
 };
 
@@ -85,8 +90,16 @@ int dfail(bimp_diff* d, int code, const std::string& m) {
             return dfail(d, BIMP_E_DEVICE, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-// Taps, tap derivatives and bank spectra of (ratio, gamma), on the device.
-int set_params(bimp_diff* d, float ratio, float gamma, hipStream_t s) {
+// Taps, tap derivatives and bank spectra of (ratio, gamma), on the device.  They replace those
+// that a forward reads, so the last one ends first: it may still run on a stream that the null
+// stream, which all of this goes to, does not wait for.  A backward has ended when its call
+// returns.
+int set_params(bimp_diff* d, float ratio, float gamma) {
+    const hipStream_t s = nullptr;
+    if (d->fwdCaptured)
+        DCHK(d, hipDeviceSynchronize());
+    else if (d->fwdPending)
+        DCHK(d, hipStreamWaitEvent(s, d->fwdDone, 0));
     const double pi = 3.1415926535897932384626433832795;
     bimpk::TapTrig trig;
     for (int o = 0; o < kNumOri; ++o) {
@@ -110,7 +123,7 @@ int set_params(bimp_diff* d, float ratio, float gamma, hipStream_t s) {
             }
             const auto& g = d->sc[gr.first].g;
             DCHK(d, bimpk::diff_taps(set, trig, gamma, d->taps, d->tapStride, s));
-            // T is free here: no pass of this context is under way
+            // T is free here: only a backward uses it
             DCHK(d, bimpk::diff_bank_rows(set, d->taps, d->tapStride, d->kwMax, g.FW, d->adj.T,
                                           d->tw[g.FW], s));
             DCHK(d, bimpk::diff_bank_cols(set, d->adj.T, d->kwMax, g.FH, g.FW,
@@ -118,6 +131,7 @@ int set_params(bimp_diff* d, float ratio, float gamma, hipStream_t s) {
         }
     }
     DCHK(d, hipStreamSynchronize(s));
+    d->fwdPending = false;
     d->ratio = ratio;
     d->gamma = gamma;
     return BIMP_OK;
@@ -178,6 +192,39 @@ int group_forward(bimp_diff* d, int first, int n, int img0, int nb, float* resp,
         const int k0 = n * nb * q / parts, k1 = n * nb * (q + 1) / parts;
         DCHK(d, bimpk::launch_cells(cs + k0, k1 - k0, s));
     }
+    return BIMP_OK;
+}
+
+int forward(bimp_diff* d, const float* img, int nimg, float* resp, hipStream_t s) {
+    const size_t isz = (size_t)d->width * d->height;
+    // chunks of images whose pyramids fit d->lev; each group takes nbf of them per launch
+    for (int b0 = 0; b0 < nimg; b0 += d->nbMax) {
+        const int nb = std::min(d->nbMax, nimg - b0);
+        int st = pyramid(d, img + b0 * isz, nb, s);
+        if (st) return st;
+        for (const auto& gr : d->groups) {
+            const int nbf = d->sc[gr.first].nbf;
+            for (int b = 0; b < nb; b += nbf)
+                if ((st = group_forward(d, gr.first, gr.second, b, std::min(nbf, nb - b),
+                                        resp + (size_t)(b0 + b) * d->respSize, s)))
+                    return st;
+        }
+    }
+    return BIMP_OK;
+}
+
+// What a parameter change has to wait for: the work that a forward has put on s.  (Nothing on the
+// null stream, where the change itself runs: the marker, a barrier packet, takes 3 us.)
+int mark_forward(bimp_diff* d, hipStream_t s) {
+    if (!s) return BIMP_OK;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    DCHK(d, hipStreamIsCapturing(s, &capturing));
+    if (capturing != hipStreamCaptureStatusNone) {
+        d->fwdCaptured = true;
+        return BIMP_OK;
+    }
+    DCHK(d, hipEventRecord(d->fwdDone, s));
+    d->fwdPending = true;
     return BIMP_OK;
 }
 
@@ -361,8 +408,12 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
         if (hipMemcpy(p, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess)
             return bail(BIMP_E_DEVICE);
     }
+    // (orders kernels of this device only)
+    if (hipEventCreateWithFlags(&d->fwdDone,
+                                hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess)
+        return bail(BIMP_E_ALLOC);
     if (bimpk::prepare_common() != hipSuccess) return bail(BIMP_E_DEVICE);
-    const int st = set_params(d, d->opt.sigma_ratio, d->opt.gamma, nullptr);
+    const int st = set_params(d, d->opt.sigma_ratio, d->opt.gamma);
     if (st) return bail(st);
     *out = d;
     return BIMP_OK;
@@ -385,6 +436,7 @@ int bimp_diff_destroy(bimp_diff* d) {
                     (void*)d->adj.C, (void*)d->adj.gm, (void*)d->adj.Yc, (void*)d->taps,
                     (void*)d->maxslot, (void*)d->partials, (void*)d->R, (void*)d->T, (void*)d->Sf})
         (void)hipFree(p);
+    if (d->fwdDone) (void)hipEventDestroy(d->fwdDone);
     delete d;
     return BIMP_OK;
 }
@@ -394,28 +446,16 @@ long long bimp_diff_response_size(const bimp_diff* d) { return d ? (long long)d-
 int bimp_diff_set_params(bimp_diff* d, float sigma_ratio, float gamma) {
     if (!d || !(sigma_ratio > 0.f) || !(gamma > 0.f)) return BIMP_E_ARG;
     if (sigma_ratio == d->ratio && gamma == d->gamma) return BIMP_OK;
-    return set_params(d, sigma_ratio, gamma, nullptr);
+    return set_params(d, sigma_ratio, gamma);
 }
 
 int bimp_diff_forward(bimp_diff* d, const float* d_img, int nimg, float* d_resp,
                       bimp_stream_t stream) {
     if (!d || !d_img || !d_resp || nimg <= 0) return BIMP_E_ARG;
-    hipStream_t s = (hipStream_t)stream;
-    const size_t isz = (size_t)d->width * d->height;
-    // chunks of images whose pyramids fit d->lev; each group takes nbf of them per launch
-    for (int b0 = 0; b0 < nimg; b0 += d->nbMax) {
-        const int nb = std::min(d->nbMax, nimg - b0);
-        int st = pyramid(d, d_img + b0 * isz, nb, s);
-        if (st) return st;
-        for (const auto& gr : d->groups) {
-            const int nbf = d->sc[gr.first].nbf;
-            for (int b = 0; b < nb; b += nbf)
-                if ((st = group_forward(d, gr.first, gr.second, b, std::min(nbf, nb - b),
-                                        d_resp + (size_t)(b0 + b) * d->respSize, s)))
-                    return st;
-        }
-    }
-    return BIMP_OK;
+    const hipStream_t s = (hipStream_t)stream;
+    const int st = forward(d, d_img, nimg, d_resp, s);
+    const int marked = mark_forward(d, s);  // after a failure too: some of it may be under way
+    return st ? st : marked;
 }
 
 int bimp_diff_backward(bimp_diff* d, const float* d_img, int nimg, const float* d_grad_resp,

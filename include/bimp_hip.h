@@ -398,10 +398,12 @@ const char* bimp_batch_last_error(const bimp_batch* batch);
  * gives the uint8 path's maps up to the pyramid's rounding; levels above 0 use the float
  * pyramid).  Responses are nimg x bimp_diff_response_size() floats: the D maps of the scales in
  * ascending wavelength order, each data_h x data_w.  The Gabor parameters (sigma ratio, gamma)
- * start at opt's values.  The backward pass recomputes the complex responses, writes
- * d(loss)/d(image) for an upstream gradient of the responses, and the gradient with respect to
- * (sigma ratio, gamma) summed over the images into grad_params (host, 2 doubles).  It
- * synchronises the stream. */
+ * start at opt's values; bimp_diff_set_params waits for the context's last forward, whatever its
+ * stream (and, once a forward has been captured into a graph, for the device, since the library
+ * does not see the replays), and returns when the new bank is in place.  The backward pass
+ * recomputes the complex responses, writes d(loss)/d(image) for an upstream gradient of the
+ * responses, and the gradient with respect to (sigma ratio, gamma) summed over the images into
+ * grad_params (host, 2 doubles).  It synchronises the stream. */
 typedef struct bimp_diff bimp_diff;
 int bimp_diff_create(int width, int height, const float* lambdas, int n, const bimp_options* opt,
                      bimp_diff** out);
