@@ -288,6 +288,19 @@ __global__ void __launch_bounds__(256) k_knn2(const float* __restrict__ q, int n
     }
 }
 
+// Whether 64-bit minima work on p: memory of the current device.  Host memory that the device can
+// write takes plain stores but no such atomics (PCIe carries only add, swap and compare-and-swap),
+// and managed or another device's memory is not relied on either.
+bool device_atomics(const void* p) {
+    int dev = -1;
+    hipPointerAttribute_t a{};
+    if (hipGetDevice(&dev) != hipSuccess || hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();  // not an address that the runtime knows
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && !a.isManaged && a.device == dev;
+}
+
 template <int R, bool VEC>
 void launch_knn2(const float* q, int nq, int qld, const float* t, int nt, int tld, int dim,
                  int* idx2, float* dist2, hipStream_t s) {
@@ -296,8 +309,9 @@ void launch_knn2(const float* q, int nq, int qld, const float* t, int nt, int tl
     // One tile per workgroup up to 4096 workgroups, then slices of several tiles (8000 x 8000:
     // 32 slices 479 us, 8 slices 552 us; 4000 x 4000: 63 slices 131 us, 8 slices 177 us; 517 x
     // 433: 14 slices 16 us, one 119 us).  The outputs hold the slices' keys only where they are
-    // 8-byte aligned; otherwise a query has one slice.
-    const bool keys = ((uintptr_t)idx2 | (uintptr_t)dist2) % 8 == 0;
+    // 8-byte aligned and in this device's memory; otherwise a query has one slice.
+    const bool keys = ntiles > 1 && ((uintptr_t)idx2 | (uintptr_t)dist2) % 8 == 0 &&
+                      device_atomics(idx2) && device_atomics(dist2);
     int per = std::max(1, ntiles);
     if (keys) per = std::max(1, (int)(((long)ntiles * nqt + 4095) / 4096));
     // (a grid's y extent is limited to 65535)

@@ -350,7 +350,10 @@ int bimp_surf_descriptors(const unsigned* d_integral, int width, int height, con
  * rows (q_ld floats apart) the two train rows (t_ld apart) with the smallest distances,
  * sqrt of the FP32 sum of squared differences over dim dimensions in order; ties go to the
  * lower train index.  d_idx2 / d_dist2 get 2 entries per query (index -1 and +inf when there
- * is no second row).  No synchronisation. */
+ * is no second row).  Where both are 8-byte aligned memory of the current device, parts of the
+ * train set are searched side by side and meet there, several times faster; any other memory that
+ * the device can write, or 4-byte alignment, gives the same results from one pass per query.  No
+ * synchronisation. */
 int bimp_match_knn2(const float* d_query, int nq, int q_ld, const float* d_train, int nt,
                     int t_ld, int dim, int* d_idx2, float* d_dist2, bimp_stream_t stream);
 /* downloadMatches (bimp.cpp:208-240), host memory: query i keeps (i, idx2[2i], 0, dist2[2i])
