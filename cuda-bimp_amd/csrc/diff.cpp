@@ -351,7 +351,10 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
     // of the padded size, the gradient's pairs and, per orientation, two complex and one real
     // map) stay within 4 GB.  More pairs mean fewer and longer launches: eight 512 x 512 images
     // took 2277, 2084 and 2017 us with 8, 16 and 32, five 200 x 130 images 616, 479 and 350 us.
+    // A launch holds no more than one group's scales of the images held at once.
     size_t pm = 0, kwfw = 0;
+    int widest = 0;
+    for (const auto& gr : d->groups) widest = std::max(widest, gr.second);
     for (const auto& x : d->sc) {
         pm = std::max(pm, (size_t)x.g.FH * x.g.FW);
         kwfw = std::max(kwfw, (size_t)x.g.FW);
@@ -359,7 +362,8 @@ int bimp_diff_create(int width, int height, const float* lambdas, int n, const b
     }
     const size_t per = pm * (2 * sizeof(float2) + sizeof(uint2) +
                              kNumOri * (2 * sizeof(float2) + sizeof(float)));
-    d->entries = (int)std::max<size_t>(1, std::min<size_t>(32, (size_t(4) << 30) / per));
+    const size_t most = std::min<size_t>(32, (size_t)widest * d->nbMax);
+    d->entries = (int)std::max<size_t>(1, std::min<size_t>(most, (size_t(4) << 30) / per));
     const size_t NE = (size_t)d->entries;
     const size_t NB = (size_t)d->nbMax;
     d->lev.assign(d->maxLevel + 1, nullptr);
