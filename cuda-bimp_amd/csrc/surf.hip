@@ -208,7 +208,8 @@ __device__ __forceinline__ int round_away(float v) { return (int)roundf(v); }
 
 // Haar responses of half side h at (px, py): dx = the h x 2h box right of the sample minus the
 // one left of it, dy = the box below minus the box above, boxes clipped to the frame.  The four
-// boxes share the eight outer points of a 3 x 3 grid (an empty clipped box sums to 0 by itself).
+// boxes share the eight outer points of a 3 x 3 grid (an empty clipped box sums to 0 by itself; so
+// that the boxes of a position beyond the integers are empty ones too, the sums saturate).
 // OFF: byte offsets from the uniform base, 32 bits for an integral of up to 2^30 entries.
 template <class OFF>
 __device__ __forceinline__ void haar(const unsigned* __restrict__ ii, int W, int H, int px, int py,
@@ -217,9 +218,11 @@ __device__ __forceinline__ void haar(const unsigned* __restrict__ ii, int W, int
     auto at = [&](OFF o) {
         return *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(ii) + o);
     };
+    auto lo = [&](int p) { return __builtin_elementwise_sub_sat(p, h); };
+    auto hi = [&](int p) { return __builtin_elementwise_add_sat(p, h); };
     const OFF ld = 4 * ((OFF)W + 1);
-    const OFF c0 = (OFF)4 * clip(px - h, W), c1 = (OFF)4 * clip(px, W), c2 = (OFF)4 * clip(px + h, W);
-    const OFF r0 = clip(py - h, H) * ld, r1 = clip(py, H) * ld, r2 = clip(py + h, H) * ld;
+    const OFF c0 = (OFF)4 * clip(lo(px), W), c1 = (OFF)4 * clip(px, W), c2 = (OFF)4 * clip(hi(px), W);
+    const OFF r0 = clip(lo(py), H) * ld, r1 = clip(py, H) * ld, r2 = clip(hi(py), H) * ld;
     const unsigned a00 = at(r0 + c0), a01 = at(r0 + c1), a02 = at(r0 + c2);
     const unsigned a10 = at(r1 + c0), a12 = at(r1 + c2);
     const unsigned a20 = at(r2 + c0), a21 = at(r2 + c1), a22 = at(r2 + c2);
