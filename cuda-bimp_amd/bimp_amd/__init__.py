@@ -498,7 +498,7 @@ def color_features(kp_matrix, bgr):
 
 def surf_descriptors(gray, kp_matrix, upright=False):
     """SURF descriptors (n x 64) and angles (n,) of the keypoints of a 7-row matrix over a gray
-    uint8 frame, on the device (integral image, then one wavefront per keypoint)."""
+    uint8 frame, on the device (integral image, then two or four keypoints per workgroup)."""
     gray = np.ascontiguousarray(gray, np.uint8)
     mat = np.ascontiguousarray(kp_matrix, np.float32)
     h, w = gray.shape

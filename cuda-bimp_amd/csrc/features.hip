@@ -66,11 +66,12 @@ __global__ void __launch_bounds__(64) k_color_features(const float* __restrict__
 // time, dimension-major, in two buffers: the next piece is loaded into registers while the
 // current one is used, one barrier per piece.
 //
-// Bound: FP32 VALU, one subtraction and one fma per query, train and dimension (no packed
-// FP32; the matrix cores' |q|^2 + |t|^2 - 2qt would lose the small distances' digits): 8000 x
-// 8000 x 152 takes 0.44 ms back to back, no more than these operations alone take at 2.4 GHz.
-// R = 4 takes two 16-byte LDS reads per 32 of them.  Before, one
-// workgroup walked the whole train set for its 64 queries, in one LDS buffer: 125 workgroups
+// Bound: FP32 VALU issue, one subtraction and one fma per query, train and dimension (no packed
+// FP32; the matrix cores' |q|^2 + |t|^2 - 2qt would lose the small distances' digits).  A loop of
+// nothing but such instructions on registers issues 73 T lanes/s, so 8000 x 8000 x 152 cannot take
+// less than 0.27 ms; the kernel's 369 M wavefront instructions would take 0.32 ms and it takes
+// 0.43 to 0.46 (boxes differ), with two 16-byte LDS reads per 32 operations beside them.  Before,
+// one workgroup walked the whole train set for its 64 queries, in one LDS buffer: 125 workgroups
 // for 8000 queries, 3.66 ms; 517 x 433 x 152 took 177 us on 9 workgroups, now 16 us.
 constexpr int kDC = 16;
 
@@ -307,8 +308,8 @@ void launch_knn2(const float* q, int nq, int qld, const float* t, int nt, int tl
     constexpr int K = 16 * R;
     const int ntiles = (nt + K - 1) / K, nqt = (nq + K - 1) / K;
     // One tile per workgroup up to 4096 workgroups, then slices of several tiles (8000 x 8000:
-    // 32 slices 479 us, 8 slices 552 us; 4000 x 4000: 63 slices 131 us, 8 slices 177 us; 517 x
-    // 433: 14 slices 16 us, one 119 us).  The outputs hold the slices' keys only where they are
+    // 32 slices 465 us, 16 477, 8 519, one 2436; 4000 x 4000: 63 slices 128 us, 8 slices 167;
+    // 517 x 433: 14 slices 16 us, one 118).  The outputs hold the slices' keys only where they are
     // 8-byte aligned and in this device's memory; otherwise a query has one slice.
     const bool keys = ntiles > 1 && ((uintptr_t)idx2 | (uintptr_t)dist2) % 8 == 0 &&
                       device_atomics(idx2) && device_atomics(dist2);
@@ -332,8 +333,8 @@ void dispatch_knn2(const float* q, int nq, int qld, const float* t, int nt, int 
                    int* idx2, float* dist2, hipStream_t s) {
     // R = 4 where its tiles fill the chip's 256 CUs a few times over (it runs six workgroups
     // per CU), else R = 2, whose tiles are four times as many: 2000 x 2000 x 152 (1024 tiles of
-    // 64 x 64) 45 us against 57 us with R = 2, 1000 x 1000 (256 tiles) 31 against 22 us.  R = 8
-    // took 525 us against 479 us at 8000 x 8000 (211 VGPRs, two wavefronts per SIMD).
+    // 64 x 64) 43 us against 52 us with R = 2, 1000 x 1000 (256 tiles) 30 against 21 us.  R = 8
+    // took a tenth longer than R = 4 at 8000 x 8000 (211 VGPRs, two wavefronts per SIMD).
     const long tiles4 = (long)((nq + 63) / 64) * ((nt + 63) / 64);
     if (tiles4 >= 768)
         launch_knn2<4, VEC>(q, nq, qld, t, nt, tld, dim, idx2, dist2, s);

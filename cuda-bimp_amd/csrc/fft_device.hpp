@@ -4,8 +4,9 @@
 // wavefront per vector; TPV = 128 for 4096: two wavefronts, so that a lane keeps 32 values and
 // not 64); every lane keeps E = N/TPV complex values in registers.  Each
 // radix-R stage does E/R butterflies per lane entirely in registers; between stages the
-// group exchanges data through its own LDS region (N floats: real parts, then imaginary
-// parts), so the only cross-lane traffic is one LDS write + read per stage boundary.
+// group exchanges data through its own LDS region (fft_lds_floats<N>() floats: real parts, then
+// imaginary parts), one LDS write + read per stage boundary; the first boundary of 512, 1536,
+// 2048, 2560, 3072 and 3584 points is a transpose between lanes and registers instead (kRegFirst).
 //
 // Index maps (Stockham autosort, radix list R0..RL, Ns = product of earlier radices):
 //   stage input  of butterfly j = lane + TPV*m, leg r : j + r*N/R

@@ -210,7 +210,8 @@ __device__ __forceinline__ int round_away(float v) { return (int)roundf(v); }
 // one left of it, dy = the box below minus the box above, boxes clipped to the frame.  The four
 // boxes share the eight outer points of a 3 x 3 grid (an empty clipped box sums to 0 by itself; so
 // that the boxes of a position beyond the integers are empty ones too, the sums saturate).
-// OFF: byte offsets from the uniform base, 32 bits for an integral of up to 2^30 entries.
+// OFF: byte offsets from the uniform base, 32 bits for an integral of up to 2^30 entries (all that
+// bimp_integral_image makes; a caller's own may be larger).
 template <class OFF>
 __device__ __forceinline__ void haar(const unsigned* __restrict__ ii, int W, int H, int px, int py,
                                      int h, float* dx, float* dy) {
